@@ -34,6 +34,11 @@ C_ABI_SYMBOLS = (
     "crumpet_fused_swin_attention_shifted",
     "crumpet_window_qkv_3d",
     "crumpet_window_proj_3d",
+    "crumpet_swin_mlp",
+    "crumpet_swin_mlp_fits",
+    "crumpet_rows_norm",
+    "crumpet_merge_norm_3d",
+    "crumpet_rows_linear",
 )
 
 OP_NAMES = (
@@ -49,6 +54,9 @@ OP_NAMES = (
     "window_qkv_3d",
     "window_proj_3d",
     "window_msa_3d",
+    "swin_mlp",
+    "patch_merge_3d",
+    "channel_norm",
 )
 
 _hip = None
@@ -79,7 +87,7 @@ def _load() -> None:
 
 
 def _mutating_op_fake(*args, **kwargs) -> None:
-    """The crumpet_ops ops other than window_msa_3d write into a
+    """The crumpet_ops ops other than those of _RETURNING_FAKES write into a
     caller-allocated output and return nothing, so their fake (meta) kernel
     has nothing to do."""
     return None
@@ -93,11 +101,32 @@ def _window_msa_fake(x, norm_weight, norm_bias, eps, w_qkv, b_qkv, w_proj, b_pro
     return x.new_empty((B, D, H, W, w_proj.shape[0]), dtype=w_qkv.dtype)
 
 
+def _swin_mlp_fake(x, add, norm_weight, norm_bias, eps, w1, b1, w2, b2):
+    return x.new_empty(x.shape)
+
+
+def _patch_merge_fake(x, norm_weight, norm_bias, eps, weight, order):
+    B, D, H, W, _ = x.shape
+    return x.new_empty((B, (D + 1) // 2, (H + 1) // 2, (W + 1) // 2, weight.shape[0]), dtype=weight.dtype)
+
+
+def _channel_norm_fake(x, weight, bias, eps, dtype):
+    return x.new_empty(x.shape, dtype=dtype)
+
+
+_RETURNING_FAKES = {
+    "window_msa_3d": _window_msa_fake,
+    "swin_mlp": _swin_mlp_fake,
+    "patch_merge_3d": _patch_merge_fake,
+    "channel_norm": _channel_norm_fake,
+}
+
+
 def _declare_fake_kernels() -> None:
     """Fake kernels for FakeTensor / torch.compile tracing of the ops (the
     reference registers the same no-op fakes: torch-ext/crumpet/__init__.py:50-73)."""
     for name in OP_NAMES:
-        fake = _window_msa_fake if name == "window_msa_3d" else _mutating_op_fake
+        fake = _RETURNING_FAKES.get(name, _mutating_op_fake)
         try:
             torch.library.register_fake(f"crumpet_ops::{name}")(fake)
         except (RuntimeError, ValueError):

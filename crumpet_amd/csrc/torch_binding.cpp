@@ -8,7 +8,8 @@
 // `attn_mask_tiles` / `fused_swin_attention_tiled` (a 16-bit mask's tiled
 // copy and attention reading it), the fused block projections
 // `window_qkv_3d` / `window_proj_3d`, and `window_msa_3d`, which runs those
-// three kernels for a whole block half in one dispatcher call.  Every impl checks
+// three kernels for a whole block half in one dispatcher call; `swin_mlp` (the
+// block's other half), `patch_merge_3d` and `channel_norm`.  Every impl checks
 // shapes, dtypes and devices (so no launch can index outside its tensors),
 // takes the current HIP stream of the tensor's device (ROCm torch tags HIP
 // devices as "cuda", hence the masquerading guard/stream helpers) and forwards to the
@@ -422,6 +423,123 @@ at::Tensor window_msa_3d(const at::Tensor& x, const std::optional<at::Tensor>& n
     return y;
 }
 
+// LayerNorm parameters of C channels: both optional, one dtype.
+int32_t norm_params(const std::optional<at::Tensor>& weight, const std::optional<at::Tensor>& bias, int64_t C,
+                    const at::Device& dev, const void** w, const void** b, const char* what) {
+    int32_t dt = CRUMPET_DTYPE_F32;
+    *w = *b = nullptr;
+    for (const auto* p : {&weight, &bias}) {
+        if (!p->has_value()) continue;
+        const at::Tensor& t = p->value();
+        TORCH_CHECK(t.dim() == 1 && t.size(0) == C && t.is_contiguous() && t.device() == dev, what,
+                    ": LayerNorm parameters must be contiguous [C] tensors on x's device");
+        dt = dtype_code(t.scalar_type());
+        TORCH_CHECK(dt >= 0, what, ": LayerNorm parameter dtype must be float32, float16 or bfloat16");
+        *(p == &weight ? w : b) = t.data_ptr();
+    }
+    if (weight.has_value() && bias.has_value())
+        TORCH_CHECK(weight->scalar_type() == bias->scalar_type(), what,
+                    ": LayerNorm weight and bias must share a dtype");
+    return dt;
+}
+
+const void* ptr_or_null(const std::optional<at::Tensor>& t) { return t.has_value() ? t->data_ptr() : nullptr; }
+
+// The second half of a Swin block, x1 + MLP(LN(x1)) with x1 = x + add, over
+// the rows of x [..., C]: one kernel where both weights fit the LDS
+// (crumpet_swin_mlp_fits), else the norm and the two projections with the
+// normalised rows, the hidden layer and x1 allocated here.
+at::Tensor swin_mlp(const at::Tensor& x, const std::optional<at::Tensor>& add,
+                    const std::optional<at::Tensor>& norm_weight, const std::optional<at::Tensor>& norm_bias,
+                    double eps, const at::Tensor& w1, const std::optional<at::Tensor>& b1, const at::Tensor& w2,
+                    const std::optional<at::Tensor>& b2) {
+    const char* what = "swin_mlp";
+    TORCH_CHECK(x.dim() >= 1 && x.is_cuda() && x.is_contiguous(), what,
+                ": x must be a contiguous tensor on a HIP device");
+    const int64_t C = x.size(-1), rows = C > 0 ? x.numel() / C : 0;
+    TORCH_CHECK(w1.dim() == 2, what, ": w1 must have shape [hidden, C]");
+    const int64_t hidden = w1.size(0);
+    const int32_t xdt = dtype_code(x.scalar_type()), dt = dtype_code(w1.scalar_type());
+    TORCH_CHECK(xdt >= 0 && dt >= 0, what, ": dtypes must be float32, float16 or bfloat16");
+    check_linear_params(w1, b1, C, w1.scalar_type(), x.device(), what);
+    check_linear_params(w2, b2, hidden, w1.scalar_type(), x.device(), what);
+    TORCH_CHECK(w2.size(0) == C, what, ": w2 must have shape [C, hidden]");
+    if (add.has_value())
+        TORCH_CHECK(add->sizes() == x.sizes() && add->is_contiguous() && add->device() == x.device() &&
+                        add->scalar_type() == w1.scalar_type(),
+                    what, ": add must be a contiguous tensor like x in the weights' dtype");
+    const void *lw, *lb;
+    const int32_t ldt = norm_params(norm_weight, norm_bias, C, x.device(), &lw, &lb, what);
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    at::Tensor y = at::empty(x.sizes(), x.options());
+    if (rows == 0) return y;
+    void* s = stream_of(x);
+    if (crumpet_swin_mlp_fits(C, hidden)) {
+        check_status(crumpet_swin_mlp(y.data_ptr(), x.data_ptr(), xdt, ptr_or_null(add), dt, rows, C, hidden, lw, lb,
+                                      ldt, static_cast<float>(eps), w1.data_ptr(), ptr_or_null(b1), w2.data_ptr(),
+                                      ptr_or_null(b2), s));
+        return y;
+    }
+    const auto opts = x.options().dtype(w1.scalar_type());
+    at::Tensor a = at::empty({rows, C}, opts), h = at::empty({rows, hidden}, opts);
+    at::Tensor x1 = add.has_value() ? at::empty(x.sizes(), x.options()) : x;
+    check_status(crumpet_rows_norm(a.data_ptr(), dt, add.has_value() ? x1.data_ptr() : nullptr, x.data_ptr(), xdt,
+                                   ptr_or_null(add), dt, rows, C, lw, lb, ldt, static_cast<float>(eps), s));
+    check_status(crumpet_rows_linear(h.data_ptr(), dt, a.data_ptr(), dt, rows, C, w1.data_ptr(), ptr_or_null(b1),
+                                     hidden, 1, nullptr, s));
+    check_status(crumpet_rows_linear(y.data_ptr(), xdt, h.data_ptr(), dt, rows, hidden, w2.data_ptr(),
+                                     ptr_or_null(b2), C, 0, x1.data_ptr(), s));
+    return y;
+}
+
+// Swin patch merging: gather and LayerNorm of the 2x2x2 neighbourhoods, then
+// the reduction, [B, D, H, W, C] -> [B, D/2, H/2, W/2, n_out].
+at::Tensor patch_merge_3d(const at::Tensor& x, const std::optional<at::Tensor>& norm_weight,
+                          const std::optional<at::Tensor>& norm_bias, double eps, const at::Tensor& weight,
+                          int64_t order) {
+    const char* what = "patch_merge_3d";
+    TORCH_CHECK(x.dim() == 5 && x.is_cuda() && x.is_contiguous(), what,
+                ": x must be a contiguous [B, D, H, W, C] tensor on a HIP device");
+    const int64_t B = x.size(0), D = x.size(1), H = x.size(2), W = x.size(3), C = x.size(4);
+    const int32_t xdt = dtype_code(x.scalar_type()), dt = dtype_code(weight.scalar_type());
+    TORCH_CHECK(xdt >= 0 && dt >= 0, what, ": dtypes must be float32, float16 or bfloat16");
+    check_linear_params(weight, std::nullopt, 8 * C, weight.scalar_type(), x.device(), what);
+    TORCH_CHECK(order >= 0 && order < (int64_t(1) << 32), what, ": order takes 32 bits");
+    const void *lw, *lb;
+    const int32_t ldt = norm_params(norm_weight, norm_bias, 8 * C, x.device(), &lw, &lb, what);
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    const auto opts = x.options().dtype(weight.scalar_type());
+    const int64_t D2 = (D + 1) / 2, H2 = (H + 1) / 2, W2 = (W + 1) / 2, rows = B * D2 * H2 * W2;
+    at::Tensor y = at::empty({B, D2, H2, W2, weight.size(0)}, opts);
+    if (rows == 0) return y;
+    at::Tensor a = at::empty({rows, 8 * C}, opts);
+    void* s = stream_of(x);
+    check_status(crumpet_merge_norm_3d(a.data_ptr(), dt, x.data_ptr(), xdt, B, D, H, W, C,
+                                       static_cast<uint32_t>(order), lw, lb, ldt, static_cast<float>(eps), s));
+    check_status(crumpet_rows_linear(y.data_ptr(), dt, a.data_ptr(), dt, rows, 8 * C, weight.data_ptr(), nullptr,
+                                     weight.size(0), 0, nullptr, s));
+    return y;
+}
+
+// LayerNorm over the last axis of x [..., C], in `dtype`.
+at::Tensor channel_norm(const at::Tensor& x, const std::optional<at::Tensor>& weight,
+                        const std::optional<at::Tensor>& bias, double eps, at::ScalarType dtype) {
+    const char* what = "channel_norm";
+    TORCH_CHECK(x.dim() >= 1 && x.is_cuda() && x.is_contiguous(), what,
+                ": x must be a contiguous tensor on a HIP device");
+    const int64_t C = x.size(-1), rows = C > 0 ? x.numel() / C : 0;
+    const int32_t xdt = dtype_code(x.scalar_type()), dt = dtype_code(dtype);
+    TORCH_CHECK(xdt >= 0 && dt >= 0, what, ": dtypes must be float32, float16 or bfloat16");
+    const void *lw, *lb;
+    const int32_t ldt = norm_params(weight, bias, C, x.device(), &lw, &lb, what);
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    at::Tensor y = at::empty(x.sizes(), x.options().dtype(dtype));
+    if (rows == 0) return y;
+    check_status(crumpet_rows_norm(y.data_ptr(), dt, nullptr, x.data_ptr(), xdt, nullptr, CRUMPET_DTYPE_F32, rows, C,
+                                   lw, lb, ldt, static_cast<float>(eps), stream_of(x)));
+    return y;
+}
+
 }  // namespace
 
 TORCH_LIBRARY(crumpet_ops, ops) {
@@ -473,6 +591,17 @@ TORCH_LIBRARY(crumpet_ops, ops) {
         "Tensor? b_qkv, Tensor w_proj, Tensor? b_proj, Tensor bias, int heads, float scale, int ws_d, "
         "int ws_h, int ws_w, int ss_d, int ss_h, int ss_w) -> Tensor",
         kCrumpetOpTags);
+    ops.def(
+        "swin_mlp(Tensor x, Tensor? add, Tensor? norm_weight, Tensor? norm_bias, float eps, Tensor w1, "
+        "Tensor? b1, Tensor w2, Tensor? b2) -> Tensor",
+        kCrumpetOpTags);
+    ops.def(
+        "patch_merge_3d(Tensor x, Tensor? norm_weight, Tensor? norm_bias, float eps, Tensor weight, "
+        "int order) -> Tensor",
+        kCrumpetOpTags);
+    ops.def(
+        "channel_norm(Tensor x, Tensor? weight, Tensor? bias, float eps, ScalarType dtype) -> Tensor",
+        kCrumpetOpTags);
 }
 
 TORCH_LIBRARY_IMPL(crumpet_ops, CUDA, ops) {
@@ -488,4 +617,7 @@ TORCH_LIBRARY_IMPL(crumpet_ops, CUDA, ops) {
     ops.impl("window_qkv_3d", &window_qkv_3d);
     ops.impl("window_proj_3d", &window_proj_3d);
     ops.impl("window_msa_3d", &window_msa_3d);
+    ops.impl("swin_mlp", &swin_mlp);
+    ops.impl("patch_merge_3d", &patch_merge_3d);
+    ops.impl("channel_norm", &channel_norm);
 }

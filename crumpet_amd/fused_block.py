@@ -165,3 +165,48 @@ def fused_window_msa_3d(
     else:
         fused_swin_attention_windows(t[0], t[1], t[2], relative_position_bias, None, None, scale, ov)
     return window_proj_3d(attn.view(nwin, n, C), wp, bp, B, D, H, W, ws, ss)
+
+
+def fused_swin_mlp(
+    x: torch.Tensor,  # [..., C]
+    add: torch.Tensor | None,  # like x, in the weights' dtype
+    norm: torch.nn.LayerNorm,
+    linear1,  # torch.nn.Linear, or its (weight, bias)
+    linear2,
+    dtype: torch.dtype | None = None,
+) -> torch.Tensor:
+    """The second half of a Swin block, ``x1 + linear2(gelu(linear1(norm(x1))))``
+    with ``x1 = x + add``, in the dtype of ``x``; ``dtype`` (float16 or
+    bfloat16, by default that of ``x``) is the compute type of the Linears.
+    One kernel up to 96 channels, else three (norm, linear + GELU, linear +
+    residual).  No gradients."""
+    _check(x, "fused_swin_mlp")
+    dtype = x.dtype if dtype is None else dtype
+    w1, b1, w2, b2 = (None if t is None else t.to(dtype).contiguous()
+                      for t in (*_linear(linear1), *_linear(linear2)))
+    return _native.ops().swin_mlp(x.contiguous(), None if add is None else add.contiguous(), norm.weight, norm.bias,
+                                  float(norm.eps), w1, b1, w2, b2)
+
+
+def patch_merge_3d(
+    x: torch.Tensor,  # [B, D, H, W, C]
+    norm: torch.nn.LayerNorm,
+    weight: torch.Tensor,  # [n_out, 8 C]
+    offsets: Sequence[Sequence[int]],
+    dtype: torch.dtype | None = None,
+) -> torch.Tensor:
+    """Swin patch merging, ``[B, ceil(D/2), ceil(H/2), ceil(W/2), n_out]`` in
+    ``dtype``: the eight voxels ``offsets`` (d, h, w in 0 / 1) of every
+    2x2x2 neighbourhood (zeros past an odd axis) concatenated, normalised and
+    projected.  No gradients."""
+    _check(x, "patch_merge_3d")
+    dtype = x.dtype if dtype is None else dtype
+    order = sum((d | h << 1 | w << 2) << 4 * p for p, (d, h, w) in enumerate(offsets))
+    return _native.ops().patch_merge_3d(x.contiguous(), norm.weight, norm.bias, float(norm.eps),
+                                        weight.to(dtype).contiguous(), order)
+
+
+def channel_norm(x: torch.Tensor, eps: float = 1e-5, dtype: torch.dtype | None = None) -> torch.Tensor:
+    """LayerNorm without parameters over the last axis, in ``dtype``.  No gradients."""
+    _check(x, "channel_norm")
+    return _native.ops().channel_norm(x.contiguous(), None, None, float(eps), x.dtype if dtype is None else dtype)

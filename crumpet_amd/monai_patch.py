@@ -14,6 +14,14 @@ the originals; True / False likewise) replace
   unshift + crop in one (opt out with ``CRUMPET_DISABLE_FUSED_BLOCK=1``);
 * ``BasicLayer.forward``: channels-last stage loop with the cached
   ``compute_attn_mask_3d`` mask (reference :201-232);
+* ``SwinTransformerBlock.forward``: in inference with a 16-bit compute type
+  the residual sums, norm2 and the MLP run as ``fused_swin_mlp``;
+* the patch merging at the end of a patched ``BasicLayer``: gather, norm and
+  reduction as ``patch_merge_3d`` (same conditions);
+* ``SwinTransformer.forward``: the stages hand each other channels-last
+  volumes and the feature norm reads them in place, where the original
+  transposes to channels-first and back around every stage (the results have
+  the original's shapes and strides);
 * ``WindowAttention.forward``: the eager ``q k^T + bias + mask -> softmax
   -> @ v`` chain becomes one gfx950 kernel call (reference :117-198).  It
   falls back to the original in training mode, with attention dropout,
@@ -46,16 +54,19 @@ in-repo MONAI-compatible model used when MONAI is absent).
 
 from __future__ import annotations
 
+import ctypes
 import functools
+import itertools
 import os
 from typing import Any
 
 import torch
 import torch.nn.functional as F
+from torch.nn.modules import module as _module
 
-from . import compute_attn_mask_3d, fused_shift_partition_3d, fused_unshift_unpartition_3d
+from . import _native, compute_attn_mask_3d, fused_shift_partition_3d, fused_unshift_unpartition_3d
 from .fused_attention import fused_swin_attention_shifted, fused_swin_attention_windows
-from .fused_block import fused_window_msa_3d
+from .fused_block import channel_norm, fused_swin_mlp, fused_window_msa_3d, patch_merge_3d
 
 _STATE: dict[str, Any] = {}
 _REQUIRED = ("SwinTransformerBlock", "BasicLayer", "WindowAttention", "get_window_size")
@@ -282,28 +293,218 @@ def _patched_window_attention_forward(original):
     return forward
 
 
+# ---- what the eager modules would do beyond the values ---------------------------
+
+def _unhooked(*modules) -> bool:
+    """Whether running the modules' math without calling them goes unnoticed."""
+    return not any(m._forward_hooks or m._forward_pre_hooks for m in modules) and not (
+        _module._global_forward_hooks or _module._global_forward_pre_hooks)
+
+
+def _values_only(x: torch.Tensor, params) -> bool:
+    """Whether a pass over ``x`` needs nothing but its values: a plain HIP
+    tensor, no gradient of any kind, no function transform, no tracing."""
+    if type(x) is not torch.Tensor or x.device.type != "cuda":
+        return False
+    if torch._C._functorch.peek_interpreter_stack() is not None:
+        return False
+    if torch.autograd.forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack() > 0:
+        return False
+    return not (torch.is_grad_enabled() and (x.requires_grad or any(p.requires_grad for p in params)))
+
+
+def _half_compute(x: torch.Tensor, params) -> torch.dtype | None:
+    """The 16-bit type the Linears of ``params`` run in on ``x``, or None
+    where they run in fp32, or where the eager ops mix types in another way
+    (without autocast everything must share x's type).  Inference tensors
+    have no version counter, which the cached casts need."""
+    if any(p.is_inference() for p in params):
+        return None
+    if torch.is_autocast_enabled("cuda"):
+        dtype = torch.get_autocast_dtype("cuda")
+        plain = x.dtype in (torch.float32, dtype) and all(
+            p.dtype in (torch.float32, x.dtype) for p in params)
+    else:
+        dtype = x.dtype
+        plain = all(p.dtype == dtype for p in params)
+    return dtype if plain and dtype in (torch.float16, torch.bfloat16) else None
+
+
+def _idle(drop) -> bool:
+    """A dropout or drop-path module that passes its input through."""
+    return isinstance(drop, torch.nn.Identity) or (
+        not drop.training and (type(drop) is torch.nn.Dropout or type(drop).__name__ == "DropPath"))
+
+
+def _linear_params(*linears):
+    return [p for m in linears for p in (m.weight, m.bias) if p is not None]
+
+
+def _affine_norm(norm, c) -> bool:
+    return type(norm) is torch.nn.LayerNorm and tuple(norm.normalized_shape) == (c,)
+
+
+def _norm_params(norm):
+    return [p for p in (norm.weight, norm.bias) if p is not None]
+
+
+def _fusable_heads(attn) -> bool:
+    """Whether the attention runs fused.  Models whose head dimension is not
+    covered keep every other eager op too, and with them eager's exact bits."""
+    return attn.dim // attn.num_heads in _HEAD_DIMS and attn.attn_drop.p == 0.0 and _fused_attn_enabled()
+
+
+@functools.lru_cache(maxsize=64)
+def _one_kernel_mlp(c: int, hidden: int) -> bool:
+    f = _native.hip_library().crumpet_swin_mlp_fits
+    f.argtypes = [ctypes.c_int64, ctypes.c_int64]
+    return bool(f(c, hidden))
+
+
+def _stream(x: torch.Tensor) -> int:
+    """The current stream: a cast made on one stream may still be in flight
+    when another one asks for it, so every stream keeps its own."""
+    return torch._C._cuda_getCurrentRawStream(x.device.index)
+
+
+def _tail_dtype(block, x) -> torch.dtype | None:
+    """The compute type of a block's fused second half, or None: inference,
+    LayerNorm -> Linear -> exact GELU -> Linear with idle dropouts, sizes
+    that the kernels take (channels and hidden features multiples of 32, or
+    of 16 where one kernel covers the block)."""
+    if torch.compiler.is_compiling() or block.training or x.dim() != 5 or not _fused_block_enabled():
+        return None
+    if getattr(block, "use_checkpoint", False) or not _fusable_heads(block.attn):
+        return None
+    norm, mlp, c = block.norm2, block.mlp, x.shape[-1]
+    if type(mlp).__name__ != "MLPBlock" or not _affine_norm(norm, c):
+        return None
+    l1, l2, fn = mlp.linear1, mlp.linear2, mlp.fn
+    if type(l1) is not torch.nn.Linear or type(l2) is not torch.nn.Linear or type(fn) is not torch.nn.GELU:
+        return None
+    if fn.approximate != "none" or not (_idle(block.drop_path) and _idle(mlp.drop1) and _idle(mlp.drop2)):
+        return None
+    hidden = l1.out_features
+    if l1.in_features != c or l2.in_features != hidden or l2.out_features != c or hidden % 32 or c > 6144:
+        return None
+    if c % 32 and not _one_kernel_mlp(c, hidden):
+        return None
+    if not _unhooked(norm, mlp, l1, l2, fn, block.drop_path, mlp.drop1, mlp.drop2):
+        return None
+    params = _linear_params(l1, l2) + _norm_params(norm)
+    return _half_compute(x, params) if _values_only(x, params) else None
+
+
+def _patched_block_forward(original, swin):
+    @functools.wraps(original)
+    def forward(self, x, mask_matrix):
+        dtype = _tail_dtype(self, x)
+        if dtype is None:
+            return original(self, x, mask_matrix)
+        half = self.forward_part1(x, mask_matrix)
+        if half.dtype != dtype:
+            x = x + half
+            return x + self.forward_part2(x)
+        mlp = self.mlp
+        l1, l2 = mlp.linear1, mlp.linear2
+
+        def cast():
+            return [tuple(None if p is None else p.to(dtype).contiguous() for p in (m.weight, m.bias))
+                    for m in (l1, l2)]
+
+        w1, w2 = _cached(mlp, ("mlp", dtype, _stream(x)), _linear_params(l1, l2), cast)
+        return fused_swin_mlp(x, half, self.norm2, w1, w2, dtype)
+
+    return forward
+
+
+# sub-grid offsets (d, h, w) in concatenation order
+_MERGE_V2 = tuple(itertools.product(range(2), repeat=3))
+_MERGE_V1 = ((0, 0, 0), (1, 0, 0), (0, 1, 0), (0, 0, 1), (1, 0, 1), (0, 1, 0), (0, 0, 1), (1, 1, 1))
+
+
+def _downsample(m, x, swin):
+    """A stage's patch merging: one gather + norm pass and the reduction, or
+    the module itself."""
+    offsets = _MERGE_V1 if type(m) is getattr(swin, "PatchMerging", None) else _MERGE_V2
+    if (torch.compiler.is_compiling() or m.training or x.dim() != 5 or not _fused_block_enabled()
+            or type(m) not in (getattr(swin, "PatchMerging", None), getattr(swin, "PatchMergingV2", None))):
+        return m(x)
+    norm, red, c = m.norm, m.reduction, x.shape[-1]
+    if (type(red) is not torch.nn.Linear or red.bias is not None or red.in_features != 8 * c
+            or red.out_features % 16 or c % 4 or c > 768 or not _affine_norm(norm, 8 * c)
+            or not _unhooked(m, norm, red)):
+        return m(x)
+    params = [red.weight] + _norm_params(norm)
+    dtype = _half_compute(x, params) if _values_only(x, params) else None
+    if dtype is None:
+        return m(x)
+    weight = _cached(red, ("merge", dtype, _stream(x)), (red.weight,), lambda: red.weight.to(dtype).contiguous())
+    return patch_merge_3d(x, norm, weight, offsets, dtype)
+
+
+def _layer_channels_last(layer, x, swin):
+    """A stage on a contiguous ``[b, d, h, w, c]`` volume, channels-last out."""
+    b, d, h, w, _ = x.shape
+    window_size, shift_size = swin.get_window_size((d, h, w), layer.window_size, layer.shift_size)
+    window_size = _as_triple(window_size)
+    shift_size = _as_triple(shift_size)
+    dp = -(-d // window_size[0]) * window_size[0]
+    hp = -(-h // window_size[1]) * window_size[1]
+    wp = -(-w // window_size[2]) * window_size[2]
+    attn_mask = compute_attn_mask_3d(D=dp, H=hp, W=wp, window_size=window_size,
+                                     shift_size=shift_size, dtype=x.dtype, device=x.device)
+    setattr(attn_mask, _GEOMETRY_ATTR, (dp, hp, wp, window_size, shift_size))
+    for blk in layer.blocks:
+        x = blk(x, attn_mask)
+    x = x.view(b, d, h, w, -1)
+    if layer.downsample is not None:
+        fused = len(layer.blocks) > 0 and _fusable_heads(layer.blocks[-1].attn)
+        x = _downsample(layer.downsample, x, swin) if fused else layer.downsample(x)
+    return x
+
+
 def _patched_basic_layer_forward(original, swin):
     @functools.wraps(original)
     def forward(self, x):
         if x.dim() != 5:
             return original(self, x)
-        b, c, d, h, w = x.shape
-        window_size, shift_size = swin.get_window_size((d, h, w), self.window_size, self.shift_size)
-        window_size = _as_triple(window_size)
-        shift_size = _as_triple(shift_size)
-        x = x.permute(0, 2, 3, 4, 1).contiguous()
-        dp = -(-d // window_size[0]) * window_size[0]
-        hp = -(-h // window_size[1]) * window_size[1]
-        wp = -(-w // window_size[2]) * window_size[2]
-        attn_mask = compute_attn_mask_3d(D=dp, H=hp, W=wp, window_size=window_size,
-                                         shift_size=shift_size, dtype=x.dtype, device=x.device)
-        setattr(attn_mask, _GEOMETRY_ATTR, (dp, hp, wp, window_size, shift_size))
-        for blk in self.blocks:
-            x = blk(x, attn_mask)
-        x = x.view(b, d, h, w, -1)
-        if self.downsample is not None:
-            x = self.downsample(x)
+        x = _layer_channels_last(self, x.permute(0, 2, 3, 4, 1).contiguous(), swin)
         return x.permute(0, 4, 1, 2, 3).contiguous()
+
+    return forward
+
+
+def _channels_last_chain(model, x, normalize, swin) -> bool:
+    """Whether the encoder's stages may hand each other channels-last
+    volumes: inference on plain tensors, every stage the patched
+    ``BasicLayer`` without hooks, normalised features."""
+    if (torch.compiler.is_compiling() or model.training or not normalize or x.dim() != 5 or type(model) is not swin.SwinTransformer
+            or getattr(model, "use_v2", False) or "proj_out" in model.__dict__ or not _fused_block_enabled()):
+        return False
+    embed = model.patch_embed.embed_dim  # the widest feature is embed << num_layers
+    if embed % 8 or embed << model.num_layers > 6144:
+        return False
+    layers = [getattr(model, f"layers{i + 1}") for i in range(model.num_layers)]
+    if not all(len(m) >= 1 and type(m[0]) is swin.BasicLayer and _unhooked(m[0]) and len(m[0].blocks)
+               and _fusable_heads(m[0].blocks[0].attn) for m in layers):
+        return False
+    return _values_only(x, model.parameters())
+
+
+def _patched_transformer_forward(original, swin):
+    @functools.wraps(original)
+    def forward(self, x, normalize=True):
+        if not _channels_last_chain(self, x, normalize, swin):
+            return original(self, x, normalize)
+        x = self.pos_drop(self.patch_embed(x)).permute(0, 2, 3, 4, 1).contiguous()
+        # F.layer_norm runs and returns in fp32 under autocast
+        dtype = torch.float32 if torch.is_autocast_enabled("cuda") else None
+        outs = [channel_norm(x, dtype=dtype).permute(0, 4, 1, 2, 3)]
+        for i in range(self.num_layers):
+            x = _layer_channels_last(getattr(self, f"layers{i + 1}")[0], x, swin)
+            outs.append(channel_norm(x, dtype=dtype).permute(0, 4, 1, 2, 3))
+        return outs
 
     return forward
 
@@ -314,14 +515,20 @@ def patch_monai_swin_unetr() -> bool:
     if _STATE.get("patched"):
         return False
     saved = []
+
+    def install(cls, name, make, *args):
+        original = cls.__dict__[name]
+        saved.append((cls, name, original))
+        setattr(cls, name, make(original, *args))
+
     for swin in _swin_modules():
-        orig = (swin.SwinTransformerBlock.forward_part1, swin.BasicLayer.forward,
-                swin.WindowAttention.forward)
-        saved.append((swin, orig))
-        swin.SwinTransformerBlock.forward_part1 = _patched_forward_part1(orig[0], swin)
-        swin.BasicLayer.forward = _patched_basic_layer_forward(orig[1], swin)
+        install(swin.SwinTransformerBlock, "forward_part1", _patched_forward_part1, swin)
+        install(swin.SwinTransformerBlock, "forward", _patched_block_forward, swin)
+        install(swin.BasicLayer, "forward", _patched_basic_layer_forward, swin)
+        if hasattr(swin, "SwinTransformer"):
+            install(swin.SwinTransformer, "forward", _patched_transformer_forward, swin)
         if _fused_attn_enabled():
-            swin.WindowAttention.forward = _patched_window_attention_forward(orig[2])
+            install(swin.WindowAttention, "forward", _patched_window_attention_forward)
     _STATE.update({"patched": True, "saved": saved})
     return True
 
@@ -331,10 +538,8 @@ def unpatch_monai_swin_unetr() -> bool:
     (reference monai_patch.py:264-275)."""
     if not _STATE.get("patched"):
         return False
-    for swin, orig in _STATE["saved"]:
-        swin.SwinTransformerBlock.forward_part1 = orig[0]
-        swin.BasicLayer.forward = orig[1]
-        swin.WindowAttention.forward = orig[2]
+    for cls, name, original in _STATE["saved"]:
+        setattr(cls, name, original)
     _STATE.clear()
     return True
 

@@ -334,6 +334,65 @@ CRUMPET_API int crumpet_window_proj_3d(void* y, const void* windows, int32_t dty
                                        int64_t ss_d, int64_t ss_h, int64_t ss_w,
                                        void* stream);
 
+/*
+ * The second half of a Swin block on rows of C channels:
+ *
+ *   x1 = x + add (rounded to x_dtype; add may be NULL),
+ *   y  = x1 + gelu(LN(x1) @ w1^T + b1) @ w2^T + b2
+ *
+ * x, y [rows, C] in x_dtype; add, w1 [hidden, C], b1, w2 [C, hidden], b2 in
+ * `dtype` (float16 or bfloat16; x_dtype is the same type or float32).
+ * LayerNorm as crumpet_window_qkv_3d, the exact (erf) GELU in fp32, the
+ * hidden layer rounded to `dtype` once, fp32 accumulation, one rounding at
+ * the end.  crumpet_swin_mlp_fits(C, hidden) says which sizes one launch
+ * covers (C a multiple of 16 up to 96, both weights in 160 KB of LDS);
+ * others run as crumpet_rows_norm and two crumpet_rows_linear.  Every
+ * pointer 16-byte aligned.
+ *
+ * No counterpart in the reference, which leaves forward_part2 and the two
+ * residual sums of MONAI's SwinTransformerBlock to PyTorch.
+ */
+CRUMPET_API int crumpet_swin_mlp(void* y, const void* x, int32_t x_dtype, const void* add, int32_t dtype,
+                                 int64_t rows, int64_t C, int64_t hidden,
+                                 const void* ln_weight, const void* ln_bias, int32_t ln_dtype, float eps,
+                                 const void* w1, const void* b1, const void* w2, const void* b2,
+                                 void* stream);
+CRUMPET_API int crumpet_swin_mlp_fits(int64_t C, int64_t hidden);
+
+/*
+ * out = LN(x) over rows of C channels, or with `add` x1 = x + add (written
+ * to sum_out in x_dtype) and out = LN(x1).  out_dtype equals x_dtype or one
+ * of the two is float32; LayerNorm in fp32, its parameters optional.  C a
+ * multiple of 8 up to 6144; pointers 16-byte aligned.
+ */
+CRUMPET_API int crumpet_rows_norm(void* out, int32_t out_dtype, void* sum_out, const void* x, int32_t x_dtype,
+                                  const void* add, int32_t add_dtype, int64_t rows, int64_t C,
+                                  const void* ln_weight, const void* ln_bias, int32_t ln_dtype, float eps,
+                                  void* stream);
+
+/*
+ * The gather and LayerNorm of a Swin patch merging: row (b, d, h, w) of the
+ * halved grid (odd axes padded with zeros) holds 8 parts of C channels, part
+ * p being voxel (2d + od, 2h + oh, 2w + ow) of x [B, D, H, W, C] with
+ * od | oh << 1 | ow << 2 in bits 4p .. 4p + 2 of `order`; out [rows, 8 C] is
+ * its LayerNorm.  C a multiple of 4 up to 768; types as crumpet_rows_norm.
+ */
+CRUMPET_API int crumpet_merge_norm_3d(void* out, int32_t out_dtype, const void* x, int32_t x_dtype,
+                                      int64_t B, int64_t D, int64_t H, int64_t W, int64_t C, uint32_t order,
+                                      const void* ln_weight, const void* ln_bias, int32_t ln_dtype, float eps,
+                                      void* stream);
+
+/*
+ * out = act(x @ weight^T + bias) [+ residual]: x [rows, K], weight
+ * [n_out, K] and bias [n_out] (or NULL) in `dtype` (float16 or bfloat16),
+ * out and residual (or NULL) [rows, n_out] in out_dtype (`dtype` or
+ * float32).  activation 0: none, 1: the exact GELU.  fp32 accumulation, one
+ * rounding.  K a multiple of 32, n_out of 16; pointers 16-byte aligned.
+ */
+CRUMPET_API int crumpet_rows_linear(void* out, int32_t out_dtype, const void* x, int32_t dtype,
+                                    int64_t rows, int64_t K, const void* weight, const void* bias,
+                                    int64_t n_out, int32_t activation, const void* residual, void* stream);
+
 #ifdef __cplusplus
 } /* extern "C" */
 #endif

@@ -1,0 +1,166 @@
+"""The second half of a Swin block (fused_swin_mlp), patch merging and the
+feature norm against plain torch in 64 bits, at the edges of their tiles (16
+tokens and 16 or 32 features a tile, 32-deep steps shared by four waves), and
+the patched encoder against its eager forward.
+
+Tolerances: the results are rounded to the 16-bit type once, and so are the
+normalised rows and the hidden layer; with unit-variance rows and weights
+scaled by K^-1/2 each adds at most about one rounding (u = 2^-11 or 2^-8) of
+the largest value, so 6 u of it bounds their sum."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+import crumpet_amd
+from crumpet_amd import fused_block, monai_patch
+from crumpet_amd import swin_unetr_compat as sw
+
+pytestmark = pytest.mark.gpu
+
+U = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}
+
+
+def _close(got, want, dtype):
+    want = want.double()
+    err = (got.double() - want).abs().max().item()
+    assert err <= 6 * U[dtype] * want.abs().max().item(), err
+
+
+def _randn(g, *shape, dtype=torch.float32, std=1.0):
+    return (torch.randn(shape, generator=g) * std).to("cuda", dtype)
+
+
+def _norm(g, c, dtype):
+    norm = torch.nn.LayerNorm(c, device="cuda", dtype=dtype).requires_grad_(False)
+    norm.weight.copy_(1 + 0.1 * _randn(g, c))
+    norm.bias.copy_(0.1 * _randn(g, c))
+    return norm
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("c,hidden,rows", [(16, 32, 1), (32, 128, 17), (48, 192, 1000), (64, 256, 15), (80, 320, 33),
+                                           (96, 384, 5000), (96, 512, 40), (128, 512, 31), (192, 768, 129),
+                                           (384, 1536, 27), (768, 3072, 64), (192, 768, 13824)])
+@pytest.mark.parametrize("x_fp32,with_add,bias", [(True, True, True), (False, True, True), (False, False, False)])
+def test_swin_mlp(dev, dtype, c, hidden, rows, x_fp32, with_add, bias):
+    g = torch.Generator().manual_seed(c + rows)
+    xdt = torch.float32 if x_fp32 else dtype
+    x = _randn(g, rows, c, dtype=xdt)
+    add = _randn(g, rows, c, dtype=dtype) if with_add else None
+    norm = _norm(g, c, xdt)
+    l1 = (_randn(g, hidden, c, dtype=dtype, std=c ** -0.5), _randn(g, hidden, dtype=dtype, std=0.1) if bias else None)
+    l2 = (_randn(g, c, hidden, dtype=dtype, std=hidden ** -0.5), _randn(g, c, dtype=dtype, std=0.1) if bias else None)
+    got = fused_block.fused_swin_mlp(x, add, norm, l1, l2, dtype)
+    assert got.dtype == xdt and got.shape == x.shape
+    x1 = x if add is None else x + add
+    a = F.layer_norm(x1.double(), (c,), norm.weight.double(), norm.bias.double(), norm.eps)
+    up = lambda t: None if t is None else t.double()  # noqa: E731
+    want = x1.double() + F.linear(F.gelu(F.linear(a, up(l1[0]), up(l1[1]))), up(l2[0]), up(l2[1]))
+    _close(got, want, dtype)
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+def test_swin_mlp_spreads_what_is_not_finite(dev, value):
+    """A row with a value that is not finite is NaN, as in eager; the others stay."""
+    g = torch.Generator().manual_seed(0)
+    x = _randn(g, 40, 48, dtype=torch.float16)
+    x[7, 3] = value
+    norm = _norm(g, 48, torch.float16)
+    l1 = (_randn(g, 192, 48, dtype=torch.float16, std=0.1), None)
+    l2 = (_randn(g, 48, 192, dtype=torch.float16, std=0.1), None)
+    got = fused_block.fused_swin_mlp(x, None, norm, l1, l2)
+    assert torch.isnan(got[7]).all()
+    assert torch.isfinite(got[torch.arange(40, device="cuda") != 7]).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("dims,c", [((2, 2, 2), 8), ((5, 3, 4), 24), ((1, 1, 1), 48), ((7, 8, 9), 96), ((6, 6, 6), 384),
+                                    ((3, 4, 2), 768)])
+@pytest.mark.parametrize("kind", [sw.PatchMerging, sw.PatchMergingV2])
+def test_patch_merging(dev, monkeypatch, dtype, dims, c, kind):
+    torch.manual_seed(c)
+    m = kind(c).to(dev).eval().requires_grad_(False)
+    m.norm.weight.uniform_(0.9, 1.1)
+    x = torch.randn((2, *dims, c), device=dev).to(dtype)
+    want = m.to(torch.float64)(x.double())
+    m = m.to(torch.float32)
+    calls = []
+    monkeypatch.setattr(monai_patch, "patch_merge_3d",
+                        lambda *a: calls.append(1) or fused_block.patch_merge_3d(*a))
+    with torch.no_grad(), torch.autocast("cuda", dtype=dtype):
+        got = monai_patch._downsample(m, x, sw)
+    assert calls and got.dtype == dtype and got.shape == want.shape
+    _close(got, want, dtype)
+
+
+@pytest.mark.parametrize("c,rows", [(8, 3), (48, 1000), (96, 65), (192, 17), (768, 100), (1536, 33), (6144, 5)])
+@pytest.mark.parametrize("xdt,odt", [(torch.float32, torch.float32), (torch.float16, torch.float32),
+                                     (torch.bfloat16, torch.bfloat16)])
+def test_channel_norm(dev, c, rows, xdt, odt):
+    x = (3 + 2 * torch.randn((rows, c), generator=torch.Generator().manual_seed(c))).to(dev, xdt)
+    got = fused_block.channel_norm(x, dtype=odt)
+    want = F.layer_norm(x.double(), (c,))
+    # fp32: sums of c terms and a division, a few ulps of the largest value
+    bound = (1e-6 if odt == torch.float32 else U[odt]) * 2 * want.abs().max().item()
+    assert got.dtype == odt and (got.double() - want).abs().max().item() <= bound
+
+
+def _encoder(dev, **kw):
+    torch.manual_seed(0)
+    return sw.SwinTransformer(in_chans=1, embed_dim=48, window_size=(7, 7, 7), patch_size=(2, 2, 2),
+                              depths=(2, 2, 2, 2), num_heads=(3, 6, 12, 24), **kw).to(dev).eval()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, None])
+@pytest.mark.parametrize("downsample", ["merging", "mergingv2"])
+def test_patched_encoder(dev, dtype, downsample):
+    """Same shapes, strides, types and (to the rounding of eight blocks, an
+    eighth of which each 16-bit step may add) values as the eager encoder."""
+    m = _encoder(dev, downsample=downsample)
+    x = torch.rand((2, 1, 32, 48, 40), device=dev)
+
+    def run():
+        with torch.no_grad(), torch.autocast("cuda", dtype=dtype or torch.float16, enabled=dtype is not None):
+            return m(x)
+
+    want = run()
+    crumpet_amd.patch_monai_swin_unetr()
+    try:
+        got = run()
+    finally:
+        crumpet_amd.unpatch_monai_swin_unetr()
+    bound = 1e-4 if dtype is None else 64 * U[dtype]
+    for a, b in zip(got, want):
+        assert a.shape == b.shape and a.stride() == b.stride() and a.dtype == b.dtype
+        assert (a - b).abs().max().item() <= bound * b.abs().max().item()
+
+
+def test_patched_block_keeps_gradients_hooks_and_training(dev, monkeypatch):
+    """Where more than the values is wanted the eager second half runs."""
+    def fail(*a, **k):
+        raise AssertionError("fused second half")
+
+    monkeypatch.setattr(monai_patch, "fused_swin_mlp", fail)
+    block = sw.SwinTransformerBlock(48, 3, (4, 4, 4), (0, 0, 0)).to(dev).eval()
+    x = torch.randn((1, 8, 8, 8, 48), device=dev)
+    crumpet_amd.patch_monai_swin_unetr()
+    try:
+        with torch.autocast("cuda", dtype=torch.float16):
+            block(x, None).float().sum().backward()
+            assert block.mlp.linear1.weight.grad is not None
+            with torch.no_grad():
+                seen = []
+                handle = block.mlp.register_forward_hook(lambda *a: seen.append(1))
+                block(x, None)
+                handle.remove()
+                assert seen
+                block.mlp.drop1.train()
+                block(x, None)
+                block.mlp.drop1.eval()
+                monkeypatch.setenv("CRUMPET_DISABLE_FUSED_BLOCK", "1")
+                block(x, None)
+    finally:
+        crumpet_amd.unpatch_monai_swin_unetr()
