@@ -339,110 +339,152 @@ rows_norm_kernel(To* __restrict__ out, Tx* __restrict__ sum_out, const Tx* __res
 
 // ---- out = act(X W^T + b) [+ residual], X [T, K] in the compute type -------------
 //
-// A wave computes 16 FT features of 16 TT tokens with v_mfma_f32_16x16x32:
-// both operands come straight from L2 / L1 as 16-byte pieces of a row (no
-// LDS and no barrier in the loop), the next step's fragments requested
-// before the current products.  kSplit: the 4 waves of a workgroup share one
-// tile and take a quarter of K each, summed through LDS at the end, so that
-// few tokens (the deep stages: 27 to 1,728) still spread K = 384 .. 6144
-// over the chip and the chain of dependent loads is a quarter as long;
-// otherwise the waves take 2 x 2 neighbouring tiles.
-template <typename Tc, typename To, int FT, int TT, bool kSplit>
+// A workgroup of 4 waves computes 64 features of BT tokens, K in 64-deep
+// steps: a step's rows arrive as whole 128-byte lines (8 lanes a row) in
+// registers, kAhead steps ahead, and pass through LDS, 16-byte chunks xor'ed
+// with the row so that a fragment read (16 rows, one chunk) meets all banks.
+// (Fragments loaded straight from memory, 16 rows of 64 bytes an instruction,
+// move every line twice: 42 us against 14.7 for 13,824 x 768 -> 192 with the
+// residual; hipBLASLt's plain product takes 11.5.)
+//   S = 1, BT = 64: the waves take 2 x 2 quarters of the tile and share the
+//     staged rows, double-buffered, one barrier a step;
+//   S = 4, BT = 16: each wave stages and multiplies its own quarter of K (no
+//     barrier), so that few tokens (the deep stages: 27 to 1,728, K = 384 ..
+//     6144) fill the chip and the chain of dependent loads is a quarter as
+//     long.
+// Either way the tile is summed in LDS and leaves as whole lines of 64
+// features, bias, GELU and residual on the way.  Workgroups of one XCD
+// (xcd_chunk) take neighbouring tiles, features first, so that a row of X is
+// fetched into one L2.
+template <typename Tc, typename To, int BT, int S>
 __global__ void __launch_bounds__(256)
 rows_linear_kernel(To* __restrict__ out, const Tc* __restrict__ x, const Tc* __restrict__ w,
                    const Tc* __restrict__ bias, const To* __restrict__ res, int32_t act, uint32_t T, int32_t K,
-                   int32_t n_out, uint32_t ftiles) {
+                   int32_t n_out, uint32_t ftiles, uint32_t chunks) {
     typedef Mma2<Tc> M;
     typedef typename M::x8 X8;
+    static_assert((S == 1 && BT == 64) || (S == 4 && BT == 16), "four accumulator tiles a wave");
+    constexpr int kRows = 64 + BT;                   // staged rows: 64 of W, BT of X
+    constexpr int kLoaders = S == 1 ? 256 : 64;      // threads that stage them
+    constexpr int kLoads = kRows * 8 / kLoaders;     // 16-byte loads per thread and step
+    constexpr int kAhead = S == 1 ? 3 : 2;           // steps in flight
+    constexpr int kStage = kRows * 64;               // elements
+    constexpr int kRow = 68;                         // floats per token in the final sum: rows 4 banks apart
+    constexpr size_t kStageBytes = size_t(S == 1 ? 2 : 4) * kStage * 2;  // S = 4: one slice per wave
+    constexpr size_t kSumBytes = size_t(S) * BT * kRow * 4;
+    __shared__ __attribute__((aligned(16))) unsigned char smem[kStageBytes > kSumBytes ? kStageBytes : kSumBytes];
     const int lane = threadIdx.x & 63;
-    const int wave = threadIdx.x >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 15;
     const int g = lane >> 4;
-    // ftiles: workgroup tiles along the features, the faster index
-    uint32_t tf = blockIdx.x % ftiles, tt = blockIdx.x / ftiles;
-    int s0 = 0, s1 = K >> 5;
-    if constexpr (kSplit) {
-        const int n = s1;
-        s0 = n * wave >> 2;
-        s1 = n * (wave + 1) >> 2;
-    } else {
-        tf = tf * 2 + (wave & 1);
-        tt = tt * 2 + (wave >> 1);
+    uint32_t chunk;
+    if (!xcd_chunk(blockIdx.x, gridDim.x, chunks, chunk)) return;
+    const int f0 = static_cast<int>(chunk % ftiles) * 64;
+    const uint32_t t0 = chunk / ftiles * BT;
+    const int steps = (K + 63) >> 6;
+    const int s0 = S == 1 ? 0 : steps * wave / S;
+    const int s1 = S == 1 ? steps : steps * (wave + 1) / S;
+
+    Tc* const stage = reinterpret_cast<Tc*>(smem) + (S == 1 ? 0 : wave * kStage);
+    const int ltid = S == 1 ? threadIdx.x : lane;
+    const int lrow = ltid >> 3, lchunk = ltid & 7;
+    const Tc* src[kLoads];
+    int dst[kLoads];
+#pragma unroll
+    for (int i = 0; i < kLoads; ++i) {
+        const int r = i * (kLoaders / 8) + lrow;
+        // rows past the matrices repeat the last one; their results are not stored
+        src[i] = (r < 64 ? w + int64_t(min(f0 + r, n_out - 1)) * K
+                         : x + int64_t(min(t0 + uint32_t(r - 64), T - 1)) * K) + 8 * lchunk;
+        dst[i] = r * 64 + ((lchunk ^ (r & 7)) << 3);
     }
-    const int f0 = tf * 16 * FT;
-    const uint32_t t0 = tt * 16 * TT;
-    const Tc* wr[FT];
-    const Tc* xr[TT];
-#pragma unroll
-    for (int i = 0; i < FT; ++i) wr[i] = w + int64_t(min(f0 + 16 * i + col, n_out - 1)) * K + 8 * g;
-#pragma unroll
-    for (int i = 0; i < TT; ++i) xr[i] = x + int64_t(min(t0 + 16 * i + col, T - 1)) * K + 8 * g;
-    f32x4 acc[FT][TT];
-#pragma unroll
-    for (int i = 0; i < FT; ++i)
-#pragma unroll
-        for (int j = 0; j < TT; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    constexpr int kBatch = FT * TT >= 16 ? 1 : 3;  // 32-deep steps requested at a time
-    X8 wa[2][kBatch][FT], xa[2][kBatch][TT];
-    // Steps past s1 read the last step again; their products are skipped.
+    X8 regs[kAhead][kLoads];
     auto fetch = [&](int s, int buf) __attribute__((always_inline)) {
+        const int k = 64 * s;
+        const bool inside = s < s1 && k + 8 * lchunk < K;  // the last step may be half a step
 #pragma unroll
-        for (int u = 0; u < kBatch; ++u) {
-            const int k = 32 * min(s + u, (K >> 5) - 1);
-#pragma unroll
-            for (int i = 0; i < FT; ++i) wa[buf][u][i] = *reinterpret_cast<const X8*>(wr[i] + k);
-#pragma unroll
-            for (int i = 0; i < TT; ++i) xa[buf][u][i] = *reinterpret_cast<const X8*>(xr[i] + k);
+        for (int i = 0; i < kLoads; ++i) {
+            X8 v = {};
+            if (inside) v = *reinterpret_cast<const X8*>(src[i] + k);
+            regs[buf][i] = v;
         }
     };
-    auto mul = [&](int s, int buf) __attribute__((always_inline)) {
+    f32x4 acc[4];
 #pragma unroll
-        for (int u = 0; u < kBatch; ++u)
-            if (s + u < s1) {
-#pragma unroll
-                for (int i = 0; i < FT; ++i)
-#pragma unroll
-                    for (int j = 0; j < TT; ++j) acc[i][j] = M::mma32(wa[buf][u][i], xa[buf][u][j], acc[i][j]);
-            }
+    for (int i = 0; i < 4; ++i) acc[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    const int fa = S == 1 ? 32 * (wave & 1) : 0;    // the wave's features and tokens in the tile
+    const int ta = S == 1 ? 32 * (wave >> 1) : 0;
+    auto frag = [&](const Tc* st, int row, int u) __attribute__((always_inline)) {
+        return *reinterpret_cast<const X8*>(st + row * 64 + (((4 * u + g) ^ (row & 7)) << 3));
     };
-    fetch(s0, 0);
-    for (int s = s0; s < s1; s += 2 * kBatch) {
-        fetch(s + kBatch, 1);
-        mul(s, 0);
-        fetch(s + 2 * kBatch, 0);
-        mul(s + kBatch, 1);
+#pragma unroll
+    for (int d = 0; d < kAhead; ++d) fetch(s0 + d, d);
+    int buf = 0;
+    for (int s = s0; s < s1; s += kAhead) {
+#pragma unroll
+        for (int d = 0; d < kAhead; ++d) {
+            if (s + d < s1) {
+                Tc* const st = stage + (S == 1 ? buf * kStage : 0);
+#pragma unroll
+                for (int i = 0; i < kLoads; ++i) *reinterpret_cast<X8*>(st + dst[i]) = regs[d][i];
+                fetch(s + d + kAhead, d);
+                if constexpr (S == 1) {
+                    __syncthreads();
+                } else {
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                }
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    if constexpr (S == 1) {
+                        const X8 w0 = frag(st, fa + col, u), w1 = frag(st, fa + 16 + col, u);
+                        const X8 x0 = frag(st, 64 + ta + col, u), x1 = frag(st, 64 + ta + 16 + col, u);
+                        acc[0] = M::mma32(w0, x0, acc[0]);
+                        acc[1] = M::mma32(w1, x0, acc[1]);
+                        acc[2] = M::mma32(w0, x1, acc[2]);
+                        acc[3] = M::mma32(w1, x1, acc[3]);
+                    } else {
+                        const X8 x0 = frag(st, 64 + col, u);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) acc[i] = M::mma32(frag(st, 16 * i + col, u), x0, acc[i]);
+                    }
+                }
+                if constexpr (S != 1) {
+                    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                    __builtin_amdgcn_wave_barrier();
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                }
+                buf ^= 1;
+            }
+        }
     }
 
-    auto finish = [&](f32x4 v, int i, int j) __attribute__((always_inline)) {
-        const int f = f0 + 16 * i + 4 * g;
-        const uint32_t t = t0 + 16 * j + col;
-        if (f >= n_out || t >= T) return;
-        if (bias != nullptr) v += load4f(bias + f);
+    __syncthreads();  // the sums reuse the staged rows' LDS
+    float* const sum = reinterpret_cast<float*>(smem);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int f = fa + (S == 1 ? 16 * (i & 1) : 16 * i) + 4 * g;
+        const int t = ta + (S == 1 ? 16 * (i >> 1) : 0) + col;
+        *reinterpret_cast<f32x4*>(sum + ((S == 1 ? 0 : wave * BT) + t) * kRow + f) = acc[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < BT / 16; ++i) {
+        const int tok = i * 16 + (threadIdx.x >> 4), f = (threadIdx.x & 15) * 4;
+        f32x4 v = *reinterpret_cast<const f32x4*>(sum + tok * kRow + f);
+#pragma unroll
+        for (int p = 1; p < S; ++p) v += *reinterpret_cast<const f32x4*>(sum + (p * BT + tok) * kRow + f);
+        const uint32_t t = t0 + tok;
+        if (f0 + f >= n_out || t >= T) continue;
+        if (bias != nullptr) v += load4f(bias + f0 + f);
         if (act) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[e] = gelu(v[e]);
         }
-        const int64_t at = int64_t(t) * n_out + f;
+        const int64_t at = int64_t(t) * n_out + f0 + f;
         if (res != nullptr) v += load4f(res + at);
         store4f(out + at, v);
-    };
-    if constexpr (kSplit) {
-        static_assert(FT * TT == 4, "one tile per wave in the final sum");
-        __shared__ f32x4 part[4][4][64];
-#pragma unroll
-        for (int i = 0; i < FT; ++i)
-#pragma unroll
-            for (int j = 0; j < TT; ++j) part[wave][i * TT + j][lane] = acc[i][j];
-        __syncthreads();
-        f32x4 v = part[0][wave][lane];
-#pragma unroll
-        for (int p = 1; p < 4; ++p) v += part[p][wave][lane];
-        finish(v, wave / TT, wave % TT);
-    } else {
-#pragma unroll
-        for (int i = 0; i < FT; ++i)
-#pragma unroll
-            for (int j = 0; j < TT; ++j) finish(acc[i][j], i, j);
     }
 }
 
@@ -565,20 +607,16 @@ int check_norm(const char* what, int64_t rows, int64_t C, int32_t x_dtype, int32
 template <typename Tc, typename To>
 void launch_linear(hipStream_t s, void* out, const void* x, const void* w, const void* bias, const void* res,
                    int32_t act, uint32_t T, int32_t K, int32_t n_out) {
-#define CRUMPET_LINEAR(F, N, SPLIT, FTILES, TTILES)                                                            \
-    hipLaunchKernelGGL((rows_linear_kernel<Tc, To, F, N, SPLIT>), dim3((FTILES) * (TTILES)), dim3(256), 0, s,  \
-                       static_cast<To*>(out), static_cast<const Tc*>(x), static_cast<const Tc*>(w),            \
-                       static_cast<const Tc*>(bias), static_cast<const To*>(res), act, T, K, n_out, FTILES)
     const auto up = [](uint32_t a, uint32_t b) { return (a + b - 1) / b; };
-    const uint32_t n = static_cast<uint32_t>(n_out);
-    // 64 x 64 tiles per wave once they give every SIMD one; then 32 x 32
-    // tiles, K split over the waves until the tiles alone fill the chip
-    if (uint64_t(up(n, 64)) * up(T, 64) >= 1024)
-        CRUMPET_LINEAR(4, 4, false, up(n, 128), up(T, 128));
-    else if (uint64_t(up(n, 32)) * up(T, 32) >= 2048)
-        CRUMPET_LINEAR(2, 2, false, up(n, 64), up(T, 64));
+    const uint32_t ft = up(static_cast<uint32_t>(n_out), 64);
+#define CRUMPET_LINEAR(BT, S)                                                                                 do {                                                                                                          const uint32_t chunks = ft * up(T, BT);                                                                   hipLaunchKernelGGL((rows_linear_kernel<Tc, To, BT, S>), dim3(xcd_launch_count(chunks)), dim3(256),                            0, s, static_cast<To*>(out), static_cast<const Tc*>(x),                                                   static_cast<const Tc*>(w), static_cast<const Tc*>(bias),                                                  static_cast<const To*>(res), act, T, K, n_out, ft, chunks);                        } while (0)
+    // 64-token tiles once there are about three for every four CUs (216 x 768
+    // -> 3072, 192 tiles: 8.5 us against 9.5 with 16-token tiles; 1,728 x
+    // 1536 -> 384, 162 tiles: 13.0 against 12.0)
+    if (ft * up(T, 64) >= 192)
+        CRUMPET_LINEAR(64, 1);
     else
-        CRUMPET_LINEAR(2, 2, true, up(n, 32), up(T, 32));
+        CRUMPET_LINEAR(16, 4);
 #undef CRUMPET_LINEAR
 }
 
