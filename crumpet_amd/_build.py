@@ -35,6 +35,7 @@ ARCH = "gfx950"
 HIP_SOURCES = [
     "api.hip", "partition.hip", "attn_mask.hip", "mask_tile.hip", "attention.hip",
     "attention_f16.hip", "attention_bf16.hip", "attention_f32.hip", "attention_d32.hip", "attention_wide.hip",
+    "attention_chunk.hip",
     "window_linear.hip", "block_tail.hip",
 ]
 

@@ -217,6 +217,18 @@ int run_attention(const char* what, void* out, const int64_t out_strides[4], con
     for (int i = 0; i < 3; ++i) {
         if (((N - 1) * st[i][2] + 32) * esize >= (int64_t(1) << 31)) tuned32 = false;
     }
+    // head dims 32, 64 and 128 of 16-bit types with 16-byte aligned q, k and
+    // v rows run the chunk kernel, the rest of `wide` the general one
+    if (wide && !tuned32 && vec && dtype != CRUMPET_DTYPE_F32 && (Dh == 32 || Dh == 64 || Dh == 128)) {
+        bool rows16 = true;
+        for (int i = 0; i < 3; ++i)
+            if (st[i][0] % 8 || st[i][1] % 8 || st[i][2] % 8 || reinterpret_cast<uintptr_t>(ptr[i]) % 16)
+                rows16 = false;
+        if (rows16) {
+            attn::launch_chunk(p, static_cast<int>(Dh), kmask, dtype, mask_dtype, s);
+            return check_launch(what);
+        }
+    }
     if (wide && !tuned32) {
         attn::launch_wide(p, static_cast<int>(Dh), kmask, dtype, mask_dtype, s);
         return check_launch(what);

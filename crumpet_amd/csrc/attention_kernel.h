@@ -216,6 +216,9 @@ constexpr bool d32_group_slots(int NT, int strips) {
 constexpr int kWideMaxRegionN = 2048;
 constexpr int kWideQueries = 64;  // queries per workgroup of the general kernel
 void launch_wide(const Params& p, int Dh, int kmask, int32_t dtype, int32_t mask_dtype, hipStream_t s);
+// The same for 16-bit types at head dims 32, 64 and 128 with unit d stride,
+// q, k and v rows aligned to 16 bytes and out rows to 8 (attention_chunk.hip).
+void launch_chunk(const Params& p, int Dh, int kmask, int32_t dtype, int32_t mask_dtype, hipStream_t s);
 
 // Tile counts the kernel is compiled for; a call runs with the smallest one
 // that covers ceil(N / 16).

@@ -1,0 +1,83 @@
+"""The chunk attention kernel (16-bit types, head dims 32, 64 and 128, rows
+16-byte aligned) against the general kernel, which the same values take when
+their rows lie 8 bytes off, at the edges of its chunks (64 keys, 64 or 128
+queries a workgroup) in every mask mode and bias type.
+
+Tolerance: the two differ in where P and the row sum are rounded; each is held
+to the type's bound against the fp32 formula (2e-3 / 1e-2), so to twice that
+of each other."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+import crumpet_amd
+from crumpet_amd.fused_attention import fused_swin_attention, fused_swin_attention_shifted
+from helpers import TOL
+
+pytestmark = pytest.mark.gpu
+
+
+def _off(t):
+    """The same values with rows 8 bytes past 16-byte alignment."""
+    flat = torch.empty(t.numel() + 4, dtype=t.dtype, device=t.device)[4:]
+    return flat.view(t.shape).copy_(t)
+
+
+def _both(call, q, k, v, dtype):
+    a = call(q, k, v)
+    b = call(_off(q), _off(k), _off(v))
+    assert torch.isfinite(a).all()
+    assert (a.float() - b.float()).abs().max().item() <= 2 * TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("Dh", [32, 64, 128])
+@pytest.mark.parametrize("N", [1, 15, 63, 64, 65, 127, 128, 129, 192, 353, 385, 512])
+@pytest.mark.parametrize("mask_dtype,bias_dtype", [(None, torch.float32), (torch.float16, torch.bfloat16),
+                                                   (torch.float32, torch.float16), (torch.bfloat16, torch.float32)])
+def test_edges(dev, dtype, Dh, N, mask_dtype, bias_dtype):
+    g = torch.Generator(device="cuda").manual_seed(N + Dh)
+    q, k, v = (torch.randn((3, 2, N, Dh), generator=g, device="cuda").to(dtype) for _ in range(3))
+    bias = torch.randn((2, N, N), generator=g, device="cuda").to(bias_dtype)
+    mask = flags = None
+    if mask_dtype is not None:
+        mask = torch.where(torch.rand((3, N, N), generator=g, device="cuda") < 0.3, -100.0, 0.0).to(mask_dtype)
+        mask[:, :, N // 2] = 0
+        flags = torch.tensor([1, 0, 1], dtype=torch.uint8, device="cuda")
+    _both(lambda q, k, v: fused_swin_attention(q, k, v, bias, mask, flags), q, k, v, dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("Dh", [32, 64, 128])
+@pytest.mark.parametrize("ws,grid,shift", [((4, 4, 4), (2, 3, 1), (2, 2, 2)), ((3, 5, 4), (2, 2, 2), (1, 0, 2)),
+                                           ((8, 8, 8), (1, 2, 2), (4, 4, 4)), ((7, 7, 7), (2, 1, 2), (3, 3, 3))])
+def test_regions(dev, dtype, Dh, ws, grid, shift):
+    g = torch.Generator(device="cuda").manual_seed(Dh)
+    N, nw = ws[0] * ws[1] * ws[2], grid[0] * grid[1] * grid[2]
+    dims = tuple(n * w for n, w in zip(grid, ws))
+    q, k, v = (torch.randn((2 * nw, 3, N, Dh), generator=g, device="cuda").to(dtype) for _ in range(3))
+    bias = torch.randn((3, N, N), generator=g, device="cuda")
+    mask = crumpet_amd.compute_attn_mask_3d(*dims, ws, shift, torch.float32, "cuda").repeat(2, 1, 1)
+    got = fused_swin_attention_shifted(q, k, v, bias, dims, ws, shift)
+    want = fused_swin_attention(_off(q), _off(k), _off(v), bias, mask)
+    assert (got.float() - want.float()).abs().max().item() <= 2 * TOL[dtype]
+
+
+@pytest.mark.parametrize("mask_dtype", [torch.float16, torch.bfloat16, torch.float32])
+def test_lowest_and_infinite_masks(dev, mask_dtype):
+    """Keys masked by the type's lowest value or -inf, whole chunks of them
+    first: they have no part in the result."""
+    g = torch.Generator(device="cuda").manual_seed(1)
+    N = 200
+    q, k, v = (torch.randn((2, 2, N, 64), generator=g, device="cuda").half() for _ in range(3))
+    bias = torch.randn((2, N, N), generator=g, device="cuda")
+    keep = torch.arange(N, device="cuda") >= 130
+    want = torch.softmax((q.double() / 8) @ k.double()[:, :, keep].transpose(-2, -1).contiguous()
+                         + bias.double()[:, :, keep], -1) @ v.double()[:, :, keep].contiguous()
+    for low in (torch.finfo(mask_dtype).min, float("-inf")):
+        mask = torch.zeros((2, N, N), dtype=mask_dtype, device="cuda")
+        mask[:, :, ~keep] = low
+        got = fused_swin_attention(q, k, v, bias, mask)
+        assert (got.double() - want).abs().max().item() <= TOL[torch.float16]
