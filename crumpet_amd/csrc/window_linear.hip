@@ -37,8 +37,10 @@
 // independent persistent waves with the weights in registers (stage 0: 74%
 // and 77% of HBM against 60% and 69% for the tiled kernels, whose
 // workgroups drain the memory queue at every barrier).  window_qkv at C = 96
-// and 192 (stages 1 and 2) takes window_qkv_stream_lds_kernel: the same
-// persistent waves, with the weights in LDS.
+// and 192 (stages 1 and 2) with many tokens takes
+// window_qkv_stream_lds_kernel: the same persistent waves, with the weights
+// in LDS.  Other multiples of 32 channels from 96 up, and few tokens, take
+// window_rows_kernel; the tiled kernels keep fp32 and the remaining widths.
 //
 // Numerics: LayerNorm in fp32 (two passes: mean, then the mean of squared
 // deviations; biased variance, as torch), the normalised value rounded once
@@ -938,6 +940,185 @@ window_qkv_stream_lds_kernel(Tc* __restrict__ out, const Tx* __restrict__ x, con
     }
 }
 
+// Both projections for 2-byte types at C a multiple of 32 from 96 to 384, 32
+// tokens and 64 features a workgroup (qkv: LayerNorm over the gathered rows;
+// proj: the inverse gather).  The tiled kernels above are bound by their chain
+// of round trips at the deep stages (LayerNorm parameters one load at a time,
+// rows, then weights in 32-byte pieces of 16 rows).  Here:
+//   - everything a workgroup needs is requested at once: 8 lanes take a
+//     token's row as whole lines, and each wave the 16 weight rows of its
+//     features, 64-deep steps of whole lines, before the LayerNorm;
+//   - rows and weights pass through LDS (16-byte pieces xor'ed with the row),
+//     the weights through a wave's own two-step slice without a barrier, and
+//     both are the operands of v_mfma_f32_16x16x32;
+//   - LayerNorm parameters come through LDS as floats;
+//   - results leave through LDS as whole lines.
+// kQkv: rows are the padded, shifted, partitioned volume x (Tx) and out the
+// windows; else rows are windows (Tc) and out the volume.
+template <typename T>
+struct Mma32;
+template <>
+struct Mma32<_Float16> {
+    typedef _Float16 x8 __attribute__((ext_vector_type(8)));
+    static __device__ __forceinline__ f32x4 step(x8 a, x8 b, f32x4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
+    }
+};
+template <>
+struct Mma32<__bf16> {
+    typedef __bf16 x8 __attribute__((ext_vector_type(8)));
+    static __device__ __forceinline__ f32x4 step(x8 a, x8 b, f32x4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
+    }
+};
+
+template <typename Tx, typename Tc, int NK, bool kQkv>
+__global__ void __launch_bounds__(kThreads)
+window_rows_kernel(Tc* __restrict__ out, const Tx* __restrict__ x, const void* ln_w, const void* ln_b,
+                   int32_t ln_dtype, int32_t normalize, float eps, const Tc* __restrict__ w,
+                   const Tc* __restrict__ bias, int32_t C, int32_t n_out, const WinGeom g, uint32_t ftiles,
+                   uint32_t chunks) {
+    typedef typename Mma32<Tc>::x8 X8;
+    constexpr int BT = 32;                // tokens
+    constexpr int CP = 64 * NK;           // channels rounded up to whole steps
+    constexpr int kRow = 68;              // floats per token of the result
+    constexpr int kABytes = BT * CP * 2;
+    constexpr int kOBytes = BT * kRow * 4;
+    __shared__ __attribute__((aligned(16))) unsigned char smem[kABytes > kOBytes ? kABytes : kOBytes];
+    __shared__ __attribute__((aligned(16))) Tc w_lds[4][2][16 * 64];
+    __shared__ __attribute__((aligned(16))) float ln_lds[kQkv ? 2 : 1][kQkv ? CP : 4];
+    Tc* const a_lds = reinterpret_cast<Tc*>(smem);
+    uint32_t chunk;
+    if (!xcd_chunk(blockIdx.x, gridDim.x, chunks, chunk)) return;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col = lane & 15;
+    const int q = lane >> 4;
+    const int f0 = static_cast<int>(chunk % ftiles) * 64;
+    const uint32_t t0 = chunk / ftiles * BT;
+    const uint32_t T = kQkv ? g.tokens : g.vtokens;
+
+    // the token's row: lane part p of 8 holds the channels 8 (p + 8 j) .. + 7
+    const int tok = threadIdx.x >> 3;
+    const int part = threadIdx.x & 7;
+    const uint32_t t = t0 + tok;
+    uint32_t row = kPadRow;
+    if (t < T) row = kQkv ? token_row(t, g) : window_token(t, g);
+    const Tx* xr = x + int64_t(row == kPadRow ? 0 : row) * C;
+    typedef Tx TX8 __attribute__((ext_vector_type(8)));
+    TX8 xv[NK];
+#pragma unroll
+    for (int j = 0; j < NK; ++j) {
+        const int c = 8 * (part + 8 * j);
+        TX8 v = {};
+        if (row != kPadRow && c < C) v = *reinterpret_cast<const TX8*>(xr + c);
+        xv[j] = v;
+    }
+    // weight rows past n_out repeat the last one (not stored)
+    X8 wv[NK][2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int r = 8 * i + (lane >> 3), c = 8 * (lane & 7);
+        const Tc* wr = w + int64_t(min(f0 + 16 * wave + r, n_out - 1)) * C;
+#pragma unroll
+        for (int s = 0; s < NK; ++s) {
+            X8 v = {};
+            if (64 * s + c < C) v = *reinterpret_cast<const X8*>(wr + 64 * s + c);
+            wv[s][i] = v;
+        }
+    }
+    if constexpr (kQkv) {
+        const int c = 4 * static_cast<int>(threadIdx.x);
+        if (c < C) {
+            *reinterpret_cast<f32x4*>(&ln_lds[0][c]) = load_param4(ln_w, ln_dtype, c, 1.0f);
+            *reinterpret_cast<f32x4*>(&ln_lds[1][c]) = load_param4(ln_b, ln_dtype, c, 0.0f);
+        }
+        __syncthreads();
+        if (normalize) {
+            float s = 0.0f;
+#pragma unroll
+            for (int j = 0; j < NK; ++j)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) s += to_f32(xv[j][e]);
+#pragma unroll
+            for (int o = 1; o < 8; o <<= 1) s += __shfl_xor(s, o, 8);
+            const float mean = s / static_cast<float>(C);
+            float v = 0.0f;
+#pragma unroll
+            for (int j = 0; j < NK; ++j)
+                if (8 * (part + 8 * j) < C) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) {
+                        const float d = to_f32(xv[j][e]) - mean;
+                        v = __builtin_fmaf(d, d, v);
+                    }
+                }
+#pragma unroll
+            for (int o = 1; o < 8; o <<= 1) v += __shfl_xor(v, o, 8);
+            const float rstd = rsqrtf(v / static_cast<float>(C) + eps);
+#pragma unroll
+            for (int j = 0; j < NK; ++j) {
+                const int cj = 8 * (part + 8 * j);
+                X8 a = {};
+                if (row != kPadRow && cj < C) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        a[e] = static_cast<Tc>(
+                            __builtin_fmaf((to_f32(xv[j][e]) - mean) * rstd, ln_lds[0][cj + e], ln_lds[1][cj + e]));
+                }
+                *reinterpret_cast<X8*>(&a_lds[tok * CP + 8 * ((part + 8 * j) ^ (tok & 7))]) = a;
+            }
+        }
+    }
+    if (!kQkv || !normalize) {
+#pragma unroll
+        for (int j = 0; j < NK; ++j) {
+            X8 a;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) a[e] = static_cast<Tc>(to_f32(xv[j][e]));
+            *reinterpret_cast<X8*>(&a_lds[tok * CP + 8 * ((part + 8 * j) ^ (tok & 7))]) = a;
+        }
+    }
+    __syncthreads();
+
+    f32x4 acc[2] = {};
+#pragma unroll
+    for (int s = 0; s < NK; ++s) {
+        Tc* const wl = w_lds[wave][s & 1];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int r = 8 * i + (lane >> 3);
+            *reinterpret_cast<X8*>(&wl[r * 64 + 8 * ((lane & 7) ^ (r & 7))]) = wv[s][i];
+        }
+        wave_lds_sync();
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int c = 4 * u + q;
+            const X8 wf = *reinterpret_cast<const X8*>(&wl[col * 64 + 8 * (c ^ (col & 7))]);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const X8 af = *reinterpret_cast<const X8*>(
+                    &a_lds[(16 * j + col) * CP + 8 * ((8 * s + c) ^ (col & 7))]);
+                acc[j] = Mma32<Tc>::step(wf, af, acc[j]);
+            }
+        }
+    }
+    __syncthreads();  // the result reuses the rows' LDS
+    float* const o_lds = reinterpret_cast<float*>(smem);
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+        *reinterpret_cast<f32x4*>(&o_lds[(16 * j + col) * kRow + 16 * wave + 4 * q]) = acc[j];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < BT / 16; ++i) {
+        const int r = 16 * i + (threadIdx.x >> 4), f = 4 * (threadIdx.x & 15);
+        if (t0 + r >= T || f0 + f >= n_out) continue;
+        f32x4 v = *reinterpret_cast<const f32x4*>(&o_lds[r * kRow + f]);
+        if (bias != nullptr) v += load4(bias + f0 + f);
+        store4(out + int64_t(t0 + r) * n_out + f0 + f, v);
+    }
+}
+
 int elem_size(int32_t dtype) {
     switch (dtype) {
         case CRUMPET_DTYPE_F32: return 4;
@@ -1222,6 +1403,53 @@ void launch_proj_stream(int KS, int FT, hipStream_t s, void* y, const void* win,
     }
 }
 
+// window_rows_kernel's sizes: C a multiple of 32 up to 384 (at least two
+// 64-deep steps), 16-bit compute type.  Against the tiled kernels, fp16, in
+// us (tokens x C, qkv / proj): 864 x 384 15.8 -> 8.4 / 10.5 -> 4.6; 5,488 x
+// 384 93 -> 29 / 13.9 -> 7.9; 87,808 x 384 619 -> 458 / 95 -> 46; 2,744 x 288
+// 30 -> 14 / 10.0 -> 5.4; 87,808 x 128 60 -> 50 / 15.9 -> 11.0; proj 87,808 x
+// 192 29.6 -> 18.5.  The streaming proj keeps 96 -> 96 (87,808 tokens: 7.5
+// against 10.0 us).
+bool rows_sizes(int32_t dtype, int64_t C) {
+    return elem_size(dtype) == 2 && C % 32 == 0 && C > 64 && C <= 384;
+}
+// qkv at C = 96 and 192: the streaming kernel with the weights in LDS needs
+// enough tokens for its 3,072 waves (2,744 x 96: 9.2 us against 5.2 here;
+// 21,952 x 96: 10.3 against 14.2; 2,744 x 192: 9.3 against 8.2; 10,976 x 192:
+// 17.9 against 18.1).
+constexpr int64_t kRowsMaxElements = int64_t(1) << 20;
+
+template <typename Tx, typename Tc, bool kQkv>
+void launch_rows(hipStream_t s, void* out, const void* x, const void* ln_w, const void* ln_b, int32_t ln_dtype,
+                 int32_t normalize, float eps, const void* w, const void* bias, int64_t C, int64_t n_out,
+                 const WinGeom& g) {
+    const uint32_t T = kQkv ? g.tokens : g.vtokens;
+    const uint32_t ft = static_cast<uint32_t>((n_out + 63) / 64);
+    const uint32_t chunks = ft * ((T + 31) / 32);
+#define CRUMPET_ROWS(K)                                                                                      \
+    hipLaunchKernelGGL((window_rows_kernel<Tx, Tc, K, kQkv>), dim3(xcd_launch_count(chunks)), dim3(kThreads), \
+                       0, s, static_cast<Tc*>(out), static_cast<const Tx*>(x), ln_w, ln_b, ln_dtype,         \
+                       normalize, eps, static_cast<const Tc*>(w), static_cast<const Tc*>(bias),              \
+                       static_cast<int32_t>(C), static_cast<int32_t>(n_out), g, ft, chunks)
+    switch ((C + 63) / 64) {
+        case 2: CRUMPET_ROWS(2); break;
+        case 3: CRUMPET_ROWS(3); break;
+        case 4: CRUMPET_ROWS(4); break;
+        default: CRUMPET_ROWS(6); break;
+    }
+#undef CRUMPET_ROWS
+}
+
+template <typename Tx>
+void launch_rows_qkv(int32_t dtype, hipStream_t s, void* out, const void* x, const void* ln_w, const void* ln_b,
+                     int32_t ln_dtype, int32_t normalize, float eps, const void* w, const void* bias, int64_t C,
+                     int64_t n_out, const WinGeom& g) {
+    if (dtype == CRUMPET_DTYPE_F16)
+        launch_rows<Tx, _Float16, true>(s, out, x, ln_w, ln_b, ln_dtype, normalize, eps, w, bias, C, n_out, g);
+    else
+        launch_rows<Tx, __bf16, true>(s, out, x, ln_w, ln_b, ln_dtype, normalize, eps, w, bias, C, n_out, g);
+}
+
 }  // namespace
 }  // namespace crumpet
 
@@ -1257,6 +1485,18 @@ extern "C" int crumpet_window_qkv_3d(void* out, int32_t dtype, const void* x, in
          reinterpret_cast<uintptr_t>(ln_weight) | reinterpret_cast<uintptr_t>(ln_bias)) % 16 != 0)
         return fail(CRUMPET_ERR_UNSUPPORTED, "%s: pointers must be 16-byte aligned", what);
     hipStream_t s = static_cast<hipStream_t>(stream);
+    if (rows_sizes(dtype, C) && (!qkv_streams_lds(dtype, C, n_out) || g.tokens * C <= kRowsMaxElements)) {
+        if (x_dtype == CRUMPET_DTYPE_F32)
+            launch_rows_qkv<float>(dtype, s, out, x, ln_weight, ln_bias, ln_dtype, normalize, eps, weight, bias, C,
+                                   n_out, g);
+        else if (x_dtype == CRUMPET_DTYPE_F16)
+            launch_rows_qkv<_Float16>(dtype, s, out, x, ln_weight, ln_bias, ln_dtype, normalize, eps, weight, bias,
+                                      C, n_out, g);
+        else
+            launch_rows_qkv<__bf16>(dtype, s, out, x, ln_weight, ln_bias, ln_dtype, normalize, eps, weight, bias, C,
+                                    n_out, g);
+        return check_launch(what);
+    }
     if (qkv_streams(dtype, C, n_out)) {
         const int KS = static_cast<int>(C / 16);
         if (x_dtype == CRUMPET_DTYPE_F32)
@@ -1315,6 +1555,15 @@ extern "C" int crumpet_window_proj_3d(void* y, const void* windows, int32_t dtyp
          reinterpret_cast<uintptr_t>(weight) | reinterpret_cast<uintptr_t>(bias)) % 16 != 0)
         return fail(CRUMPET_ERR_UNSUPPORTED, "%s: pointers must be 16-byte aligned", what);
     hipStream_t s = static_cast<hipStream_t>(stream);
+    if (rows_sizes(dtype, C) && !proj_streams(dtype, C, n_out)) {
+        if (dtype == CRUMPET_DTYPE_F16)
+            launch_rows<_Float16, _Float16, false>(s, y, windows, nullptr, nullptr, CRUMPET_DTYPE_F32, 0, 0.0f,
+                                                   weight, bias, C, n_out, g);
+        else
+            launch_rows<__bf16, __bf16, false>(s, y, windows, nullptr, nullptr, CRUMPET_DTYPE_F32, 0, 0.0f, weight,
+                                               bias, C, n_out, g);
+        return check_launch(what);
+    }
     if (proj_streams(dtype, C, n_out)) {
         const int KS = static_cast<int>(C / 16), FT = static_cast<int>(n_out / 16);
         if (dtype == CRUMPET_DTYPE_F16)
