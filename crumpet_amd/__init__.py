@@ -164,6 +164,23 @@ class _WindowPermute(torch.autograd.Function):
         return grad_src, None, None, None
 
 
+def _permute(src: torch.Tensor, grid: WindowGrid, to_windows: bool, batch: int, name: str) -> torch.Tensor:
+    """One permutation with its gradient: the native op, or the Python
+    autograd function where tracing or a function transform looks into it."""
+    ops = _device_ops(src.device, name)
+    if (torch.compiler.is_compiling() or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch.autograd.forward_ad._current_level >= 0):
+        with _op_range("crumpet." + name):
+            if torch.is_grad_enabled() and src.requires_grad:
+                return _WindowPermute.apply(src, grid, to_windows, batch)
+            src = src.contiguous()
+            return _to_windows(src, grid) if to_windows else _to_volume(src, grid, batch)
+    if os.environ.get("CRUMPET_ENABLE_NVTX", "0") == "1":
+        with _op_range("crumpet." + name):
+            return ops.window_permute_3d(src, to_windows, *grid.permute_args)
+    return ops.window_permute_3d(src, to_windows, *grid.permute_args)
+
+
 def fused_shift_partition_3d(
     x: torch.Tensor,
     window_size: Sequence[int],
@@ -181,11 +198,7 @@ def fused_shift_partition_3d(
     grid = _grid(D, H, W, window_size, shift_size)
     if x.device.type == "meta":
         return x.new_empty(grid.windows_shape(batch, channels))
-    _device_ops(x.device, "fused_shift_partition_3d")
-    with _op_range("crumpet.fused_shift_partition_3d"):
-        if torch.is_grad_enabled() and x.requires_grad:
-            return _WindowPermute.apply(x, grid, True, batch)
-        return _to_windows(x.contiguous(), grid)
+    return _permute(x, grid, True, batch, "fused_shift_partition_3d")
 
 
 def fused_unshift_unpartition_3d(
@@ -212,11 +225,7 @@ def fused_unshift_unpartition_3d(
         raise ValueError(f"windows must have shape {expected}")
     if windows.device.type == "meta":
         return windows.new_empty(grid.volume_shape(batch, channels))
-    _device_ops(windows.device, "fused_unshift_unpartition_3d")
-    with _op_range("crumpet.fused_unshift_unpartition_3d"):
-        if torch.is_grad_enabled() and windows.requires_grad:
-            return _WindowPermute.apply(windows, grid, False, batch)
-        return _to_volume(windows.contiguous(), grid, batch)
+    return _permute(windows, grid, False, batch, "fused_unshift_unpartition_3d")
 
 
 def patch_monai_swin_unetr() -> bool:

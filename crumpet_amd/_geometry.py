@@ -9,6 +9,7 @@ is the behaviour followed).
 
 from __future__ import annotations
 
+import functools
 from dataclasses import dataclass
 from typing import Sequence
 
@@ -67,6 +68,11 @@ class WindowGrid:
                     f"shift_size[{axis}] must satisfy 0 <= shift < window_size[{axis}]"
                 )
         return cls(dims, window, shift)
+
+    @functools.cached_property
+    def permute_args(self) -> tuple[int, ...]:
+        """``D, H, W`` and ``op_args``, as ``window_permute_3d`` takes them."""
+        return (*self.dims, *self.window, *self.shift)
 
     @property
     def volume(self) -> int:

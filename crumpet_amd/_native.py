@@ -54,6 +54,7 @@ OP_NAMES = (
     "window_qkv_3d",
     "window_proj_3d",
     "window_msa_3d",
+    "window_permute_3d",
     "swin_mlp",
     "patch_merge_3d",
     "channel_norm",
@@ -101,6 +102,13 @@ def _window_msa_fake(x, norm_weight, norm_bias, eps, w_qkv, b_qkv, w_proj, b_pro
     return x.new_empty((B, D, H, W, w_proj.shape[0]), dtype=w_qkv.dtype)
 
 
+def _window_permute_fake(src, to_windows, D, H, W, ws_d, ws_h, ws_w, ss_d, ss_h, ss_w):
+    n_windows, volume = (D // ws_d) * (H // ws_h) * (W // ws_w), ws_d * ws_h * ws_w
+    if to_windows:
+        return src.new_empty((src.shape[0] * n_windows, volume, src.shape[4]))
+    return src.new_empty((src.shape[0] // n_windows, D, H, W, src.shape[2]))
+
+
 def _swin_mlp_fake(x, add, norm_weight, norm_bias, eps, w1, b1, w2, b2):
     return x.new_empty(x.shape)
 
@@ -116,6 +124,7 @@ def _channel_norm_fake(x, weight, bias, eps, dtype):
 
 _RETURNING_FAKES = {
     "window_msa_3d": _window_msa_fake,
+    "window_permute_3d": _window_permute_fake,
     "swin_mlp": _swin_mlp_fake,
     "patch_merge_3d": _patch_merge_fake,
     "channel_norm": _channel_norm_fake,
