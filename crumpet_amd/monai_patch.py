@@ -296,8 +296,9 @@ def _patched_window_attention_forward(original):
 # ---- what the eager modules would do beyond the values ---------------------------
 
 def _unhooked(*modules) -> bool:
-    """Whether running the modules' math without calling them goes unnoticed."""
-    return not any(m._forward_hooks or m._forward_pre_hooks for m in modules) and not (
+    """Whether running the modules' math without calling them goes unnoticed:
+    no hooks, and no forward that a program put on the object itself."""
+    return not any(m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__ for m in modules) and not (
         _module._global_forward_hooks or _module._global_forward_pre_hooks)
 
 
@@ -317,8 +318,10 @@ def _half_compute(x: torch.Tensor, params) -> torch.dtype | None:
     """The 16-bit type the Linears of ``params`` run in on ``x``, or None
     where they run in fp32, or where the eager ops mix types in another way
     (without autocast everything must share x's type).  Inference tensors
-    have no version counter, which the cached casts need."""
-    if any(p.is_inference() for p in params):
+    have no version counter, which the cached casts need, and the kernels'
+    16-byte accesses need what eager does not, aligned storage (parameters
+    that are views of one flat vector often are not)."""
+    if any(p.is_inference() for p in params) or any(t.data_ptr() % 16 for t in (x, *params)):
         return None
     if torch.is_autocast_enabled("cuda"):
         dtype = torch.get_autocast_dtype("cuda")
@@ -351,7 +354,7 @@ def _norm_params(norm):
 def _fusable_heads(attn) -> bool:
     """Whether the attention runs fused.  Models whose head dimension is not
     covered keep every other eager op too, and with them eager's exact bits."""
-    return attn.dim // attn.num_heads in _HEAD_DIMS and attn.attn_drop.p == 0.0 and _fused_attn_enabled()
+    return _fused_attn_enabled() and attn.dim // attn.num_heads in _HEAD_DIMS and attn.attn_drop.p == 0.0
 
 
 @functools.lru_cache(maxsize=64)
