@@ -1,7 +1,9 @@
-// General fused window attention for the shapes the head-dim-16 kernel does
-// not cover: head dims 32, 64, 128 and 256, and windows of more than 512
-// tokens (any head dim of 16..256 that is a power of two, any N).  At head
-// dim 256 a wave holds about 330 registers (one wave per SIMD).  Same contract
+// General fused window attention: any head dim of 16..256 that is a power of
+// two, any N, any strides.  It runs what the bias-stationary kernel
+// (attention_kernel.h) and the chunk kernel (attention_chunk.hip) do not take:
+// fp32 at head dim 32 and up, head dim 256, head dim 16 beyond 512 tokens, and
+// 16-bit rows off the 16-byte grid.  At head dim 256 a wave holds about 330
+// registers (one wave per SIMD).  Same contract
 // and the same three mask modes as swin_attention_tuned_kernel
 // (attention_kernel.h); the numerics are the reference's:
 //
