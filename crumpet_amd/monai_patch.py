@@ -295,6 +295,16 @@ def _patched_window_attention_forward(original):
 
 # ---- what the eager modules would do beyond the values ---------------------------
 
+_HALF = (torch.float16, torch.bfloat16)
+
+
+def _computes_half(x: torch.Tensor) -> bool:
+    """Whether the fused second half and patch merging may apply at all; asked
+    first, so that an fp32 model, whose host is the slower side, pays for no
+    other check."""
+    return x.device.type == "cuda" and _compute_dtype(x) in _HALF
+
+
 def _unhooked(*modules) -> bool:
     """Whether running the modules' math without calling them goes unnoticed:
     no hooks, and no forward that a program put on the object itself."""
@@ -330,7 +340,7 @@ def _half_compute(x: torch.Tensor, params) -> torch.dtype | None:
     else:
         dtype = x.dtype
         plain = all(p.dtype == dtype for p in params)
-    return dtype if plain and dtype in (torch.float16, torch.bfloat16) else None
+    return dtype if plain and dtype in _HALF else None
 
 
 def _idle(drop) -> bool:
@@ -375,7 +385,9 @@ def _tail_dtype(block, x) -> torch.dtype | None:
     LayerNorm -> Linear -> exact GELU -> Linear with idle dropouts, sizes
     that the kernels take (channels and hidden features multiples of 32, or
     of 16 where one kernel covers the block)."""
-    if torch.compiler.is_compiling() or block.training or x.dim() != 5 or not _fused_block_enabled():
+    if torch.compiler.is_compiling() or not _computes_half(x):
+        return None
+    if block.training or x.dim() != 5 or not _fused_block_enabled():
         return None
     if getattr(block, "use_checkpoint", False) or not _fusable_heads(block.attn):
         return None
@@ -430,7 +442,8 @@ def _downsample(m, x, swin):
     """A stage's patch merging: one gather + norm pass and the reduction, or
     the module itself."""
     offsets = _MERGE_V1 if type(m) is getattr(swin, "PatchMerging", None) else _MERGE_V2
-    if (torch.compiler.is_compiling() or m.training or x.dim() != 5 or not _fused_block_enabled()
+    if (torch.compiler.is_compiling() or not _computes_half(x) or m.training or x.dim() != 5
+            or not _fused_block_enabled()
             or type(m) not in (getattr(swin, "PatchMerging", None), getattr(swin, "PatchMergingV2", None))):
         return m(x)
     norm, red, c = m.norm, m.reduction, x.shape[-1]

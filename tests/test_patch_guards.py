@@ -23,3 +23,9 @@ def test_storage_off_the_16_byte_grid_stays_eager(offset, takes, which):
     part, whole = flat[offset:offset + 48], torch.zeros(48, dtype=torch.float16)
     x, p = (part, whole) if which == "input" else (whole, part)
     assert (monai_patch._half_compute(x, [p]) is torch.float16) == takes
+
+
+@pytest.mark.parametrize("device", ["cpu", "meta"])
+def test_other_devices_are_turned_away_before_the_block_is_looked_at(device):
+    x = torch.empty((1, 2, 2, 2, 48), dtype=torch.float16, device=device)
+    assert monai_patch._tail_dtype(object(), x) is None
