@@ -109,13 +109,13 @@ def _window_permute_fake(src, to_windows, D, H, W, ws_d, ws_h, ws_w, ss_d, ss_h,
     return src.new_empty((src.shape[0] // n_windows, D, H, W, src.shape[2]))
 
 
-def _swin_mlp_fake(x, add, norm_weight, norm_bias, eps, w1, b1, w2, b2):
+def _swin_mlp_fake(x, add, norm_weight, norm_bias, eps, w1, b1, w2, b2, dtype):
     return x.new_empty(x.shape)
 
 
-def _patch_merge_fake(x, norm_weight, norm_bias, eps, weight, order):
+def _patch_merge_fake(x, norm_weight, norm_bias, eps, weight, order, dtype):
     B, D, H, W, _ = x.shape
-    return x.new_empty((B, (D + 1) // 2, (H + 1) // 2, (W + 1) // 2, weight.shape[0]), dtype=weight.dtype)
+    return x.new_empty((B, (D + 1) // 2, (H + 1) // 2, (W + 1) // 2, weight.shape[0]), dtype=dtype)
 
 
 def _channel_norm_fake(x, weight, bias, eps, dtype):

@@ -17,11 +17,16 @@
 // C ABI of libcrumpet_hip.so (include/crumpet_hip.h).  A non-OK status
 // becomes a RuntimeError carrying crumpet_last_error().
 #include <ATen/core/Tensor.h>
+#include <ATen/ops/_foreach_copy.h>
 #include <ATen/ops/empty.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/library.h>
+
+#include <array>
+#include <optional>
+#include <vector>
 
 #include "crumpet_hip.h"
 
@@ -518,17 +523,57 @@ int32_t norm_params(const std::optional<at::Tensor>& weight, const std::optional
 
 const void* ptr_or_null(const std::optional<at::Tensor>& t) { return t.has_value() ? t->data_ptr() : nullptr; }
 
+// Parameters of Linears in `dtype`: those that are in it already as they are,
+// the rest converted into one buffer (16-byte aligned pieces) by one launch.
+// On every call, so that a pass uses the parameters as they are then, however
+// they were written (a write through .data moves no version counter, and an
+// address is reused): about 9 us of host time for the four of an MLP, against
+// 20 for one conversion after the other.
+template <size_t N>
+std::array<std::optional<at::Tensor>, N> in_dtype(const std::array<const std::optional<at::Tensor>, N>& params,
+                                                  at::ScalarType dtype) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    std::array<std::optional<at::Tensor>, N> out;
+    std::vector<at::Tensor> from, to;
+    const int64_t align = 16 / static_cast<int64_t>(c10::elementSize(dtype));
+    int64_t size = 0;
+    for (size_t i = 0; i < N; ++i) {
+        if (!params[i].has_value()) continue;
+        out[i] = params[i]->scalar_type() == dtype ? params[i]->contiguous() : *params[i];
+        if (params[i]->scalar_type() != dtype) size += (params[i]->numel() + align - 1) / align * align;
+    }
+    if (size == 0) return out;
+    at::Tensor buffer;
+    int64_t at = 0;
+    for (auto& t : out) {
+        if (!t.has_value() || t->scalar_type() == dtype) continue;
+        if (!buffer.defined()) buffer = at::empty({size}, t->options().dtype(dtype));
+        from.push_back(*t);
+        to.push_back(buffer.narrow(0, at, t->numel()).view(t->sizes()));
+        at += (t->numel() + align - 1) / align * align;
+        t = to.back();
+    }
+    at::_foreach_copy_(to, from);
+    return out;
+}
+
 // The second half of a Swin block, x1 + MLP(LN(x1)) with x1 = x + add, over
-// the rows of x [..., C]: one kernel where both weights fit the LDS
-// (crumpet_swin_mlp_fits), else the norm and the two projections with the
-// normalised rows, the hidden layer and x1 allocated here.
+// the rows of x [..., C], the Linears in `dtype`: one kernel where both
+// weights fit the LDS (crumpet_swin_mlp_fits), else the norm and the two
+// projections with the normalised rows, the hidden layer and x1 allocated
+// here.
 at::Tensor swin_mlp(const at::Tensor& x, const std::optional<at::Tensor>& add,
                     const std::optional<at::Tensor>& norm_weight, const std::optional<at::Tensor>& norm_bias,
-                    double eps, const at::Tensor& w1, const std::optional<at::Tensor>& b1, const at::Tensor& w2,
-                    const std::optional<at::Tensor>& b2) {
+                    double eps, const at::Tensor& weight1, const std::optional<at::Tensor>& bias1,
+                    const at::Tensor& weight2, const std::optional<at::Tensor>& bias2, at::ScalarType dtype) {
     const char* what = "swin_mlp";
     TORCH_CHECK(x.dim() >= 1 && x.is_cuda() && x.is_contiguous(), what,
                 ": x must be a contiguous tensor on a HIP device");
+    TORCH_CHECK(dtype_code(dtype) >= 0, what, ": dtype must be float32, float16 or bfloat16");
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    const auto params = in_dtype<4>({weight1, bias1, weight2, bias2}, dtype);
+    const at::Tensor &w1 = *params[0], &w2 = *params[2];
+    const std::optional<at::Tensor>&b1 = params[1], &b2 = params[3];
     const int64_t C = x.size(-1), rows = C > 0 ? x.numel() / C : 0;
     TORCH_CHECK(w1.dim() == 2, what, ": w1 must have shape [hidden, C]");
     const int64_t hidden = w1.size(0);
@@ -543,7 +588,6 @@ at::Tensor swin_mlp(const at::Tensor& x, const std::optional<at::Tensor>& add,
                     what, ": add must be a contiguous tensor like x in the weights' dtype");
     const void *lw, *lb;
     const int32_t ldt = norm_params(norm_weight, norm_bias, C, x.device(), &lw, &lb, what);
-    const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
     at::Tensor y = at::empty(x.sizes(), x.options());
     if (rows == 0) return y;
     void* s = stream_of(x);
@@ -566,13 +610,16 @@ at::Tensor swin_mlp(const at::Tensor& x, const std::optional<at::Tensor>& add,
 }
 
 // Swin patch merging: gather and LayerNorm of the 2x2x2 neighbourhoods, then
-// the reduction, [B, D, H, W, C] -> [B, D/2, H/2, W/2, n_out].
+// the reduction in `dtype`, [B, D, H, W, C] -> [B, D/2, H/2, W/2, n_out].
 at::Tensor patch_merge_3d(const at::Tensor& x, const std::optional<at::Tensor>& norm_weight,
-                          const std::optional<at::Tensor>& norm_bias, double eps, const at::Tensor& weight,
-                          int64_t order) {
+                          const std::optional<at::Tensor>& norm_bias, double eps, const at::Tensor& reduction,
+                          int64_t order, at::ScalarType dtype) {
     const char* what = "patch_merge_3d";
     TORCH_CHECK(x.dim() == 5 && x.is_cuda() && x.is_contiguous(), what,
                 ": x must be a contiguous [B, D, H, W, C] tensor on a HIP device");
+    TORCH_CHECK(dtype_code(dtype) >= 0, what, ": dtype must be float32, float16 or bfloat16");
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+    const at::Tensor weight = *in_dtype<1>({reduction}, dtype)[0];
     const int64_t B = x.size(0), D = x.size(1), H = x.size(2), W = x.size(3), C = x.size(4);
     const int32_t xdt = dtype_code(x.scalar_type()), dt = dtype_code(weight.scalar_type());
     TORCH_CHECK(xdt >= 0 && dt >= 0, what, ": dtypes must be float32, float16 or bfloat16");
@@ -580,7 +627,6 @@ at::Tensor patch_merge_3d(const at::Tensor& x, const std::optional<at::Tensor>& 
     TORCH_CHECK(order >= 0 && order < (int64_t(1) << 32), what, ": order takes 32 bits");
     const void *lw, *lb;
     const int32_t ldt = norm_params(norm_weight, norm_bias, 8 * C, x.device(), &lw, &lb, what);
-    const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
     const auto opts = x.options().dtype(weight.scalar_type());
     const int64_t D2 = (D + 1) / 2, H2 = (H + 1) / 2, W2 = (W + 1) / 2, rows = B * D2 * H2 * W2;
     at::Tensor y = at::empty({B, D2, H2, W2, weight.size(0)}, opts);
@@ -670,11 +716,11 @@ TORCH_LIBRARY(crumpet_ops, ops) {
         kCrumpetOpTags);
     ops.def(
         "swin_mlp(Tensor x, Tensor? add, Tensor? norm_weight, Tensor? norm_bias, float eps, Tensor w1, "
-        "Tensor? b1, Tensor w2, Tensor? b2) -> Tensor",
+        "Tensor? b1, Tensor w2, Tensor? b2, ScalarType dtype) -> Tensor",
         kCrumpetOpTags);
     ops.def(
         "patch_merge_3d(Tensor x, Tensor? norm_weight, Tensor? norm_bias, float eps, Tensor weight, "
-        "int order) -> Tensor",
+        "int order, ScalarType dtype) -> Tensor",
         kCrumpetOpTags);
     ops.def(
         "channel_norm(Tensor x, Tensor? weight, Tensor? bias, float eps, ScalarType dtype) -> Tensor",

@@ -177,15 +177,14 @@ def fused_swin_mlp(
 ) -> torch.Tensor:
     """The second half of a Swin block, ``x1 + linear2(gelu(linear1(norm(x1))))``
     with ``x1 = x + add``, in the dtype of ``x``; ``dtype`` (float16 or
-    bfloat16, by default that of ``x``) is the compute type of the Linears.
+    bfloat16, by default that of ``x``) is the compute type of the Linears,
+    whose parameters are converted to it on every call where they are not.
     One kernel up to 96 channels, else three (norm, linear + GELU, linear +
     residual).  No gradients."""
     _check(x, "fused_swin_mlp")
     dtype = x.dtype if dtype is None else dtype
-    w1, b1, w2, b2 = (None if t is None else t.to(dtype).contiguous()
-                      for t in (*_linear(linear1), *_linear(linear2)))
     return _native.ops().swin_mlp(x.contiguous(), None if add is None else add.contiguous(), norm.weight, norm.bias,
-                                  float(norm.eps), w1, b1, w2, b2)
+                                  float(norm.eps), *_linear(linear1), *_linear(linear2), dtype)
 
 
 def patch_merge_3d(
@@ -202,8 +201,7 @@ def patch_merge_3d(
     _check(x, "patch_merge_3d")
     dtype = x.dtype if dtype is None else dtype
     order = sum((d | h << 1 | w << 2) << 4 * p for p, (d, h, w) in enumerate(offsets))
-    return _native.ops().patch_merge_3d(x.contiguous(), norm.weight, norm.bias, float(norm.eps),
-                                        weight.to(dtype).contiguous(), order)
+    return _native.ops().patch_merge_3d(x.contiguous(), norm.weight, norm.bias, float(norm.eps), weight, order, dtype)
 
 
 def channel_norm(x: torch.Tensor, eps: float = 1e-5, dtype: torch.dtype | None = None) -> torch.Tensor:

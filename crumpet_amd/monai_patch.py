@@ -327,11 +327,10 @@ def _values_only(x: torch.Tensor, params) -> bool:
 def _half_compute(x: torch.Tensor, params) -> torch.dtype | None:
     """The 16-bit type the Linears of ``params`` run in on ``x``, or None
     where they run in fp32, or where the eager ops mix types in another way
-    (without autocast everything must share x's type).  Inference tensors
-    have no version counter, which the cached casts need, and the kernels'
-    16-byte accesses need what eager does not, aligned storage (parameters
-    that are views of one flat vector often are not)."""
-    if any(p.is_inference() for p in params) or any(t.data_ptr() % 16 for t in (x, *params)):
+    (without autocast everything must share x's type).  The kernels' 16-byte
+    accesses need what eager does not, aligned storage (parameters that are
+    views of one flat vector often are not)."""
+    if any(t.data_ptr() % 16 for t in (x, *params)):
         return None
     if torch.is_autocast_enabled("cuda"):
         dtype = torch.get_autocast_dtype("cuda")
@@ -374,12 +373,6 @@ def _one_kernel_mlp(c: int, hidden: int) -> bool:
     return bool(f(c, hidden))
 
 
-def _stream(x: torch.Tensor) -> int:
-    """The current stream: a cast made on one stream may still be in flight
-    when another one asks for it, so every stream keeps its own."""
-    return torch._C._cuda_getCurrentRawStream(x.device.index)
-
-
 def _tail_dtype(block, x) -> torch.dtype | None:
     """The compute type of a block's fused second half, or None: inference,
     LayerNorm -> Linear -> exact GELU -> Linear with idle dropouts, sizes
@@ -420,15 +413,7 @@ def _patched_block_forward(original, swin):
         if half.dtype != dtype:
             x = x + half
             return x + self.forward_part2(x)
-        mlp = self.mlp
-        l1, l2 = mlp.linear1, mlp.linear2
-
-        def cast():
-            return [tuple(None if p is None else p.to(dtype).contiguous() for p in (m.weight, m.bias))
-                    for m in (l1, l2)]
-
-        w1, w2 = _cached(mlp, ("mlp", dtype, _stream(x)), _linear_params(l1, l2), cast)
-        return fused_swin_mlp(x, half, self.norm2, w1, w2, dtype)
+        return fused_swin_mlp(x, half, self.norm2, self.mlp.linear1, self.mlp.linear2, dtype)
 
     return forward
 
@@ -455,8 +440,7 @@ def _downsample(m, x, swin):
     dtype = _half_compute(x, params) if _values_only(x, params) else None
     if dtype is None:
         return m(x)
-    weight = _cached(red, ("merge", dtype, _stream(x)), (red.weight,), lambda: red.weight.to(dtype).contiguous())
-    return patch_merge_3d(x, norm, weight, offsets, dtype)
+    return patch_merge_3d(x, norm, red.weight, offsets, dtype)
 
 
 def _layer_channels_last(layer, x, swin):

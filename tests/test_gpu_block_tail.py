@@ -164,3 +164,71 @@ def test_patched_block_keeps_gradients_hooks_and_training(dev, monkeypatch):
                 block(x, None)
     finally:
         crumpet_amd.unpatch_monai_swin_unetr()
+
+
+def _patched(run):
+    crumpet_amd.patch_monai_swin_unetr()
+    try:
+        return run()
+    finally:
+        crumpet_amd.unpatch_monai_swin_unetr()
+
+
+def test_second_half_and_merging_follow_their_weights(dev):
+    """Every pass uses the Linears' weights as they are then: after a write
+    through .data (which moves no version counter), and with parameters that
+    a call swaps in (whose storage may be one that an earlier call freed)."""
+    torch.manual_seed(0)
+    layer = sw.BasicLayer(48, 1, 3, (4, 4, 4), 0.0, downsample=sw.PatchMerging).to(dev).eval().requires_grad_(False)
+    mlp, red = layer.blocks[0].mlp, layer.downsample.reduction
+    x = torch.randn((1, 48, 8, 8, 8), device=dev)
+
+    def both(swap=None):
+        def run():
+            with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16, cache_enabled=False):
+                return layer(x) if swap is None else torch.func.functional_call(layer, swap(), (x,))
+        return _patched(run), run()
+
+    def agree(got, want):
+        # four roundings to 16 bits on the way to the merged values, at most
+        # doubled by the norm between them
+        assert (got - want).abs().max().item() <= 8 * U[torch.float16] * want.abs().max().item()
+
+    agree(*both())
+    mlp.linear2.weight.data.mul_(3)
+    mlp.linear1.bias.data.add_(0.5)
+    agree(*both())
+    red.weight.data.copy_(red.weight.flip(0))
+    agree(*both())
+    names = [n for n, _ in layer.named_parameters() if "mlp" in n or "reduction" in n]
+    for i in range(6):
+        start = {n: p.clone() for n, p in layer.named_parameters() if n in names}
+        agree(*both(lambda: {n: p * (1 + 0.2 * i) for n, p in start.items()}))
+
+
+def test_captured_second_half_reads_the_weights_at_replay(dev):
+    torch.manual_seed(0)
+    block = sw.SwinTransformerBlock(48, 3, (4, 4, 4), (0, 0, 0)).to(dev).eval().requires_grad_(False)
+    x = torch.randn((1, 8, 8, 8, 48), device=dev)
+
+    def run():
+        with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16, cache_enabled=False):
+            return block(x, None)
+
+    def check():
+        s = torch.cuda.Stream()
+        s.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(s):
+            run()
+        torch.cuda.current_stream().wait_stream(s)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            y = run()
+        for scale in (1.0, 2.0, 0.5, 1.0):
+            block.mlp.linear2.weight.data.mul_(scale)
+            torch.randn(1 << 20, device=dev).sum().item()
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(y, run())
+
+    _patched(check)
