@@ -58,6 +58,7 @@ import ctypes
 import functools
 import itertools
 import os
+import sys
 from typing import Any
 
 import torch
@@ -312,6 +313,22 @@ def _unhooked(*modules) -> bool:
         _module._global_forward_hooks or _module._global_forward_pre_hooks)
 
 
+@functools.lru_cache(maxsize=None)
+def _own(cls, name):
+    """``cls.name`` as the module that defines ``cls`` wrote it; None if a
+    program had put another function there when it was first asked for."""
+    method = getattr(cls, name)
+    code = getattr(method, "__code__", None)
+    source = getattr(sys.modules.get(cls.__module__), "__file__", None)
+    return method if code is not None and code.co_filename == source else None
+
+
+def _stock(obj, cls, name) -> bool:
+    """Whether ``obj.name`` is the method that ``cls``'s module wrote: not that
+    of a subclass, nor one that a program put on the class or the object."""
+    return getattr(type(obj), name, None) is _own(cls, name) and name not in obj.__dict__
+
+
 def _values_only(x: torch.Tensor, params) -> bool:
     """Whether a pass over ``x`` needs nothing but its values: a plain HIP
     tensor, no gradient of any kind, no function transform, no tracing."""
@@ -373,14 +390,19 @@ def _one_kernel_mlp(c: int, hidden: int) -> bool:
     return bool(f(c, hidden))
 
 
-def _tail_dtype(block, x) -> torch.dtype | None:
+def _tail_dtype(block, x, swin=None) -> torch.dtype | None:
     """The compute type of a block's fused second half, or None: inference,
-    LayerNorm -> Linear -> exact GELU -> Linear with idle dropouts, sizes
-    that the kernels take (channels and hidden features multiples of 32, or
-    of 16 where one kernel covers the block)."""
+    the module's own ``forward_part2`` (LayerNorm -> Linear -> exact GELU ->
+    Linear) with idle dropouts, sizes that the kernels take (channels and
+    hidden features multiples of 32, or of 16 where one kernel covers the
+    block).  ``swin`` is the patched module, by default the in-repo one."""
     if torch.compiler.is_compiling() or not _computes_half(x):
         return None
     if block.training or x.dim() != 5 or not _fused_block_enabled():
+        return None
+    if swin is None:
+        from . import swin_unetr_compat as swin
+    if not _stock(block, swin.SwinTransformerBlock, "forward_part2"):
         return None
     if getattr(block, "use_checkpoint", False) or not _fusable_heads(block.attn):
         return None
@@ -404,9 +426,11 @@ def _tail_dtype(block, x) -> torch.dtype | None:
 
 
 def _patched_block_forward(original, swin):
+    own = _own(swin.SwinTransformerBlock, "forward") is original
+
     @functools.wraps(original)
     def forward(self, x, mask_matrix):
-        dtype = _tail_dtype(self, x)
+        dtype = _tail_dtype(self, x, swin) if own else None
         if dtype is None:
             return original(self, x, mask_matrix)
         half = self.forward_part1(x, mask_matrix)

@@ -6,7 +6,9 @@ from __future__ import annotations
 import pytest
 import torch
 
+import crumpet_amd
 from crumpet_amd import monai_patch
+from crumpet_amd import swin_unetr_compat as sw
 
 
 def test_a_forward_set_on_the_module_is_called():
@@ -29,3 +31,51 @@ def test_storage_off_the_16_byte_grid_stays_eager(offset, takes, which):
 def test_other_devices_are_turned_away_before_the_block_is_looked_at(device):
     x = torch.empty((1, 2, 2, 2, 48), dtype=torch.float16, device=device)
     assert monai_patch._tail_dtype(object(), x) is None
+
+
+def _fused(monkeypatch, block, c=32):
+    """Whether the block's second half would run fused on a 16-bit volume;
+    the checks that need a HIP device are answered in its place."""
+    monkeypatch.setattr(monai_patch, "_computes_half", lambda x: True)
+    monkeypatch.setattr(monai_patch, "_values_only", lambda x, params: True)
+    return monai_patch._tail_dtype(block, torch.zeros((1, 4, 4, 4, c), dtype=torch.float16)) is torch.float16
+
+
+def _block(cls=sw.SwinTransformerBlock, c=32):
+    return cls(c, c // 16, (4, 4, 4), (0, 0, 0)).half().eval().requires_grad_(False)
+
+
+class _OwnSecondHalf(sw.SwinTransformerBlock):
+    def forward_part2(self, x):
+        return x * 0
+
+
+class _OwnFirstHalf(sw.SwinTransformerBlock):
+    def forward_part1(self, x, mask_matrix):
+        return x * 0
+
+
+def test_a_second_half_of_the_programs_own_is_called(monkeypatch):
+    assert _fused(monkeypatch, _block())
+    assert _fused(monkeypatch, _block(_OwnFirstHalf))  # called either way
+    assert not _fused(monkeypatch, _block(_OwnSecondHalf))
+    block = _block()
+    block.forward_part2 = lambda x: x * 0
+    assert not _fused(monkeypatch, block)
+    stock = sw.SwinTransformerBlock.forward_part2
+    monkeypatch.setattr(sw.SwinTransformerBlock, "forward_part2", lambda self, x: stock(self, x) * 0)
+    assert not _fused(monkeypatch, _block())
+
+
+def test_a_block_forward_put_in_place_before_the_patch_stays(monkeypatch):
+    calls = []
+    monkeypatch.setattr(sw.SwinTransformerBlock, "forward", lambda self, x, mask: calls.append(1) or x)
+    monkeypatch.setattr(monai_patch, "_tail_dtype", lambda *a: pytest.fail("fused second half"))
+    monai_patch._own.cache_clear()
+    crumpet_amd.patch_monai_swin_unetr()
+    try:
+        _block()(torch.zeros((1, 4, 4, 4, 32), dtype=torch.float16), None)
+    finally:
+        crumpet_amd.unpatch_monai_swin_unetr()
+        monai_patch._own.cache_clear()
+    assert calls
