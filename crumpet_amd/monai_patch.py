@@ -313,14 +313,19 @@ def _unhooked(*modules) -> bool:
         _module._global_forward_hooks or _module._global_forward_pre_hooks)
 
 
-@functools.lru_cache(maxsize=None)
+_OWN: dict[tuple, Any] = {}
+
+
 def _own(cls, name):
-    """``cls.name`` as the module that defines ``cls`` wrote it; None if a
-    program had put another function there when it was first asked for."""
-    method = getattr(cls, name)
-    code = getattr(method, "__code__", None)
-    source = getattr(sys.modules.get(cls.__module__), "__file__", None)
-    return method if code is not None and code.co_filename == source else None
+    """``cls.name`` as the module that defines ``cls`` wrote it; None while a
+    program has another function there (unless the first was seen before)."""
+    method = _OWN.get((cls, name))
+    if method is None:
+        here = getattr(cls, name)
+        code = getattr(here, "__code__", None)
+        if code is not None and code.co_filename == getattr(sys.modules.get(cls.__module__), "__file__", None):
+            method = _OWN[cls, name] = here
+    return method
 
 
 def _stock(obj, cls, name) -> bool:
@@ -359,10 +364,19 @@ def _half_compute(x: torch.Tensor, params) -> torch.dtype | None:
     return dtype if plain and dtype in _HALF else None
 
 
-def _idle(drop) -> bool:
+def _stock_module(module, swin, *names) -> bool:
+    """Whether ``module`` is of a class that ``swin`` knows by one of
+    ``names``, with that class's own forward (a class of the same name from
+    elsewhere may compute anything)."""
+    cls = type(module)
+    return any(cls is getattr(swin, name, None) for name in names) and _stock(module, cls, "forward")
+
+
+def _idle(drop, swin) -> bool:
     """A dropout or drop-path module that passes its input through."""
-    return isinstance(drop, torch.nn.Identity) or (
-        not drop.training and (type(drop) is torch.nn.Dropout or type(drop).__name__ == "DropPath"))
+    if type(drop) is torch.nn.Identity:
+        return True
+    return not drop.training and (type(drop) is torch.nn.Dropout or _stock_module(drop, swin, "DropPath"))
 
 
 def _linear_params(*linears):
@@ -407,12 +421,14 @@ def _tail_dtype(block, x, swin=None) -> torch.dtype | None:
     if getattr(block, "use_checkpoint", False) or not _fusable_heads(block.attn):
         return None
     norm, mlp, c = block.norm2, block.mlp, x.shape[-1]
-    if type(mlp).__name__ != "MLPBlock" or not _affine_norm(norm, c):
+    # MONAI's swin_unetr imports its MLPBlock as Mlp
+    if not _stock_module(mlp, swin, "MLPBlock", "Mlp") or not _affine_norm(norm, c):
         return None
     l1, l2, fn = mlp.linear1, mlp.linear2, mlp.fn
     if type(l1) is not torch.nn.Linear or type(l2) is not torch.nn.Linear or type(fn) is not torch.nn.GELU:
         return None
-    if fn.approximate != "none" or not (_idle(block.drop_path) and _idle(mlp.drop1) and _idle(mlp.drop2)):
+    if fn.approximate != "none" or not all(
+            _idle(m, swin) for m in (block.drop_path, mlp.drop1, mlp.drop2)):
         return None
     hidden = l1.out_features
     if l1.in_features != c or l2.in_features != hidden or l2.out_features != c or hidden % 32 or c > 6144:

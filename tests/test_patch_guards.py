@@ -71,11 +71,42 @@ def test_a_block_forward_put_in_place_before_the_patch_stays(monkeypatch):
     calls = []
     monkeypatch.setattr(sw.SwinTransformerBlock, "forward", lambda self, x, mask: calls.append(1) or x)
     monkeypatch.setattr(monai_patch, "_tail_dtype", lambda *a: pytest.fail("fused second half"))
-    monai_patch._own.cache_clear()
     crumpet_amd.patch_monai_swin_unetr()
     try:
         _block()(torch.zeros((1, 4, 4, 4, 32), dtype=torch.float16), None)
     finally:
         crumpet_amd.unpatch_monai_swin_unetr()
-        monai_patch._own.cache_clear()
     assert calls
+
+
+class _Scale(torch.nn.Identity):
+    def forward(self, x):
+        return 2 * x
+
+
+def _like_named(cls):
+    """Another class of the same name and attributes that computes something else."""
+    return type(cls.__name__, (cls,), {"forward": lambda self, x: x * 0})
+
+
+def test_modules_are_known_by_their_class_not_its_name(monkeypatch):
+    block = _block()
+    block.mlp.__class__ = _like_named(sw.MLPBlock)
+    assert type(block.mlp).__name__ == "MLPBlock" and not _fused(monkeypatch, block)
+    block = _block()
+    monkeypatch.setattr(sw.MLPBlock, "forward", lambda self, x: x * 0)
+    assert not _fused(monkeypatch, block)
+    monkeypatch.undo()
+    block.drop_path = _Scale()
+    assert not _fused(monkeypatch, block)
+    block.drop_path = type("DropPath", (torch.nn.Module,), {"forward": lambda self, x: x * 0})().eval()
+    assert not _fused(monkeypatch, block)
+    monkeypatch.setattr(sw, "DropPath", _OwnDropPath, raising=False)
+    block.drop_path = _OwnDropPath().eval()
+    assert _fused(monkeypatch, block)
+    assert not _fused(monkeypatch, block.train())
+
+
+class _OwnDropPath(torch.nn.Module):
+    def forward(self, x):
+        return x
