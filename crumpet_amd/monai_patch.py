@@ -522,14 +522,21 @@ def _channels_last_chain(model, x, normalize, swin) -> bool:
     if (torch.compiler.is_compiling() or model.training or not normalize or x.dim() != 5 or type(model) is not swin.SwinTransformer
             or getattr(model, "use_v2", False) or "proj_out" in model.__dict__ or not _fused_block_enabled()):
         return False
-    embed = model.patch_embed.embed_dim  # the widest feature is embed << num_layers
-    if embed % 8 or embed << model.num_layers > 6144:
-        return False
-    layers = [getattr(model, f"layers{i + 1}") for i in range(model.num_layers)]
+    layers = [getattr(model, f"layers{i + 1}", ()) for i in range(model.num_layers)]
     if not all(len(m) >= 1 and type(m[0]) is swin.BasicLayer and _unhooked(m[0]) and len(m[0].blocks)
                and _fusable_heads(m[0].blocks[0].attn) for m in layers):
         return False
     return _values_only(x, model.parameters())
+
+
+def _feature(x):
+    """The normalised feature, channels-first, of a channels-last volume."""
+    # F.layer_norm runs and returns in fp32 under autocast
+    dtype = torch.float32 if torch.is_autocast_enabled("cuda") else None
+    c = x.shape[-1]
+    fits = c % 8 == 0 and c <= 6144 and x.data_ptr() % 16 == 0  # the kernel's rows
+    x = channel_norm(x, dtype=dtype) if fits else F.layer_norm(x, (c,))
+    return x.permute(0, 4, 1, 2, 3)
 
 
 def _patched_transformer_forward(original, swin):
@@ -538,12 +545,10 @@ def _patched_transformer_forward(original, swin):
         if not _channels_last_chain(self, x, normalize, swin):
             return original(self, x, normalize)
         x = self.pos_drop(self.patch_embed(x)).permute(0, 2, 3, 4, 1).contiguous()
-        # F.layer_norm runs and returns in fp32 under autocast
-        dtype = torch.float32 if torch.is_autocast_enabled("cuda") else None
-        outs = [channel_norm(x, dtype=dtype).permute(0, 4, 1, 2, 3)]
+        outs = [_feature(x)]
         for i in range(self.num_layers):
             x = _layer_channels_last(getattr(self, f"layers{i + 1}")[0], x, swin)
-            outs.append(channel_norm(x, dtype=dtype).permute(0, 4, 1, 2, 3))
+            outs.append(_feature(x))
         return outs
 
     return forward

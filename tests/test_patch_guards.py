@@ -110,3 +110,39 @@ def test_modules_are_known_by_their_class_not_its_name(monkeypatch):
 class _OwnDropPath(torch.nn.Module):
     def forward(self, x):
         return x
+
+
+def _encoder():
+    return sw.SwinTransformer(in_chans=1, embed_dim=32, window_size=(4, 4, 4), patch_size=(2, 2, 2), depths=(1, 1),
+                              num_heads=(2, 4)).eval().requires_grad_(False)
+
+
+def _chained(monkeypatch, model):
+    monkeypatch.setattr(monai_patch, "_values_only", lambda x, params: True)
+    return monai_patch._channels_last_chain(model, torch.zeros((1, 1, 16, 16, 16)), True, sw)
+
+
+class _Embed(torch.nn.Module):
+    """A patch embedding of a program's own: any width, no attributes."""
+
+    def __init__(self, width):
+        super().__init__()
+        self.width = width
+
+    def forward(self, x):
+        return torch.nn.functional.avg_pool3d(x, 2).expand(-1, self.width, -1, -1, -1)
+
+
+def test_a_patch_embedding_of_the_programs_own(monkeypatch):
+    crumpet_amd.patch_monai_swin_unetr()
+    try:
+        model = _encoder()
+        model.patch_embed = _Embed(32)
+        assert _chained(monkeypatch, model)
+        # widths that the norm kernel does not take go through F.layer_norm
+        x = torch.randn((1, 2, 3, 4, 30))
+        want = torch.nn.functional.layer_norm(x, (30,)).permute(0, 4, 1, 2, 3)
+        got = monai_patch._feature(x)
+        assert torch.equal(got, want) and got.stride() == want.stride()
+    finally:
+        crumpet_amd.unpatch_monai_swin_unetr()
