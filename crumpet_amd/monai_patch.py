@@ -468,8 +468,7 @@ def _downsample(m, x, swin):
     the module itself."""
     offsets = _MERGE_V1 if type(m) is getattr(swin, "PatchMerging", None) else _MERGE_V2
     if (torch.compiler.is_compiling() or not _computes_half(x) or m.training or x.dim() != 5
-            or not _fused_block_enabled()
-            or type(m) not in (getattr(swin, "PatchMerging", None), getattr(swin, "PatchMergingV2", None))):
+            or not _fused_block_enabled() or not _stock_module(m, swin, "PatchMerging", "PatchMergingV2")):
         return m(x)
     norm, red, c = m.norm, m.reduction, x.shape[-1]
     if (type(red) is not torch.nn.Linear or red.bias is not None or red.in_features != 8 * c
@@ -517,12 +516,15 @@ def _patched_basic_layer_forward(original, swin):
 
 def _channels_last_chain(model, x, normalize, swin) -> bool:
     """Whether the encoder's stages may hand each other channels-last
-    volumes: inference on plain tensors, every stage the patched
-    ``BasicLayer`` without hooks, normalised features."""
+    volumes: inference on plain tensors, the module's own ``proj_out``, every
+    stage the patched ``BasicLayer`` without hooks, normalised features."""
     if (torch.compiler.is_compiling() or model.training or not normalize or x.dim() != 5 or type(model) is not swin.SwinTransformer
-            or getattr(model, "use_v2", False) or "proj_out" in model.__dict__ or not _fused_block_enabled()):
+            or getattr(model, "use_v2", False) or not _stock(model, swin.SwinTransformer, "proj_out")
+            or not _fused_block_enabled()):
         return False
     layers = [getattr(model, f"layers{i + 1}", ()) for i in range(model.num_layers)]
+    if swin.BasicLayer.forward is not _STATE.get("basic_layer", {}).get(swin.BasicLayer):
+        return False
     if not all(len(m) >= 1 and type(m[0]) is swin.BasicLayer and _unhooked(m[0]) and len(m[0].blocks)
                and _fusable_heads(m[0].blocks[0].attn) for m in layers):
         return False
@@ -540,9 +542,11 @@ def _feature(x):
 
 
 def _patched_transformer_forward(original, swin):
+    own = _own(swin.SwinTransformer, "forward") is original
+
     @functools.wraps(original)
     def forward(self, x, normalize=True):
-        if not _channels_last_chain(self, x, normalize, swin):
+        if not (own and _channels_last_chain(self, x, normalize, swin)):
             return original(self, x, normalize)
         x = self.pos_drop(self.patch_embed(x)).permute(0, 2, 3, 4, 1).contiguous()
         outs = [_feature(x)]
@@ -560,6 +564,7 @@ def patch_monai_swin_unetr() -> bool:
     if _STATE.get("patched"):
         return False
     saved = []
+    basic_layer = {}
 
     def install(cls, name, make, *args):
         original = cls.__dict__[name]
@@ -570,11 +575,12 @@ def patch_monai_swin_unetr() -> bool:
         install(swin.SwinTransformerBlock, "forward_part1", _patched_forward_part1, swin)
         install(swin.SwinTransformerBlock, "forward", _patched_block_forward, swin)
         install(swin.BasicLayer, "forward", _patched_basic_layer_forward, swin)
+        basic_layer[swin.BasicLayer] = swin.BasicLayer.forward
         if hasattr(swin, "SwinTransformer"):
             install(swin.SwinTransformer, "forward", _patched_transformer_forward, swin)
         if _fused_attn_enabled():
             install(swin.WindowAttention, "forward", _patched_window_attention_forward)
-    _STATE.update({"patched": True, "saved": saved})
+    _STATE.update({"patched": True, "saved": saved, "basic_layer": basic_layer})
     return True
 
 

@@ -146,3 +146,34 @@ def test_a_patch_embedding_of_the_programs_own(monkeypatch):
         assert torch.equal(got, want) and got.stride() == want.stride()
     finally:
         crumpet_amd.unpatch_monai_swin_unetr()
+
+
+def test_encoder_steps_of_the_programs_own_are_called(monkeypatch):
+    crumpet_amd.patch_monai_swin_unetr()
+    try:
+        assert _chained(monkeypatch, _encoder())
+        with monkeypatch.context() as m:
+            m.setattr(sw.SwinTransformer, "proj_out", staticmethod(lambda x, normalize=False: x))
+            assert not _chained(m, _encoder())
+        with monkeypatch.context() as m:
+            m.setattr(sw.BasicLayer, "forward", lambda self, x: x)
+            assert not _chained(m, _encoder())
+        with monkeypatch.context() as m:
+            m.setattr(sw.PatchMerging, "forward", lambda self, x: "called")
+            m.setattr(monai_patch, "_computes_half", lambda x: True)
+            x = torch.zeros((1, 4, 4, 4, 32), dtype=torch.float16)
+            assert monai_patch._downsample(sw.PatchMerging(32).half().eval(), x, sw) == "called"
+    finally:
+        crumpet_amd.unpatch_monai_swin_unetr()
+
+
+def test_an_encoder_forward_put_in_place_before_the_patch_stays(monkeypatch):
+    calls = []
+    monkeypatch.setattr(sw.SwinTransformer, "forward", lambda self, x, normalize=True: calls.append(1))
+    monkeypatch.setattr(monai_patch, "_channels_last_chain", lambda *a: True)
+    crumpet_amd.patch_monai_swin_unetr()
+    try:
+        _encoder()(torch.zeros((1, 1, 16, 16, 16)))
+    finally:
+        crumpet_amd.unpatch_monai_swin_unetr()
+    assert calls
