@@ -334,14 +334,18 @@ def _stock(obj, cls, name) -> bool:
     return getattr(type(obj), name, None) is _own(cls, name) and name not in obj.__dict__
 
 
+def _watched() -> bool:
+    """Whether something follows the ops that run, and would miss those that
+    a fused kernel stands for: a function transform, forward-mode gradients,
+    a dispatch mode, torch.jit.trace."""
+    return (torch._C._functorch.peek_interpreter_stack() is not None or torch.autograd.forward_ad._current_level >= 0
+            or torch._C._len_torch_dispatch_stack() > 0 or torch.jit.is_tracing())
+
+
 def _values_only(x: torch.Tensor, params) -> bool:
     """Whether a pass over ``x`` needs nothing but its values: a plain HIP
-    tensor, no gradient of any kind, no function transform, no tracing."""
-    if type(x) is not torch.Tensor or x.device.type != "cuda":
-        return False
-    if torch._C._functorch.peek_interpreter_stack() is not None:
-        return False
-    if torch.autograd.forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack() > 0:
+    tensor, no gradient of any kind, nothing that follows the ops."""
+    if type(x) is not torch.Tensor or x.device.type != "cuda" or _watched():
         return False
     return not (torch.is_grad_enabled() and (x.requires_grad or any(p.requires_grad for p in params)))
 

@@ -232,3 +232,29 @@ def test_captured_second_half_reads_the_weights_at_replay(dev):
             assert torch.equal(y, run())
 
     _patched(check)
+
+
+def test_jit_trace_keeps_the_modules_parameters(dev):
+    """A trace of a patched block records the second half with the module's
+    parameters, not with 16-bit copies of their values at that time."""
+    torch.manual_seed(0)
+    block = sw.SwinTransformerBlock(48, 3, (4, 4, 4), (0, 0, 0)).to(dev).eval().requires_grad_(False)
+    x = torch.randn((1, 8, 8, 8, 48), device=dev)
+
+    class Alone(torch.nn.Module):
+        def __init__(self):
+            super().__init__()
+            self.block = block
+
+        def forward(self, x):
+            return self.block(x, None)
+
+    def check():
+        with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16, cache_enabled=False):
+            block(x, None)  # a pass before the trace may have kept such copies
+            traced = torch.jit.trace(Alone(), (x,), check_trace=False)
+            block.mlp.linear2.weight.mul_(3)
+            got, want = traced(x), block(x, None)
+        assert (got - want).abs().max().item() <= 6 * U[torch.float16] * want.abs().max().item()
+
+    _patched(check)

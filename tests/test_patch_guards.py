@@ -5,6 +5,7 @@ from __future__ import annotations
 
 import pytest
 import torch
+import torch.utils.flop_counter
 
 import crumpet_amd
 from crumpet_amd import monai_patch
@@ -177,3 +178,21 @@ def test_an_encoder_forward_put_in_place_before_the_patch_stays(monkeypatch):
     finally:
         crumpet_amd.unpatch_monai_swin_unetr()
     assert calls
+
+
+def test_what_follows_the_ops_sees_the_modules():
+    seen = []
+
+    def look(x):
+        seen.append(monai_patch._watched())
+        return x * 2
+
+    x = torch.ones(3)
+    look(x)
+    torch.jit.trace(look, (x,), check_trace=False)
+    torch.func.vmap(look)(x)
+    with torch.autograd.forward_ad.dual_level():
+        look(x)
+    with torch.utils.flop_counter.FlopCounterMode(display=False):
+        look(x)
+    assert seen == [False, True, True, True, True]
