@@ -388,7 +388,12 @@ def _linear_params(*linears):
 
 
 def _affine_norm(norm, c) -> bool:
-    return type(norm) is torch.nn.LayerNorm and tuple(norm.normalized_shape) == (c,)
+    """A LayerNorm over ``c`` whose parameters the kernels take: contiguous,
+    and of one type (autocast brings both to fp32, whatever they are)."""
+    if type(norm) is not torch.nn.LayerNorm or tuple(norm.normalized_shape) != (c,):
+        return False
+    params = _norm_params(norm)
+    return all(p.is_contiguous() and p.dtype == params[0].dtype for p in params)
 
 
 def _norm_params(norm):

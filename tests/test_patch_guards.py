@@ -196,3 +196,32 @@ def test_what_follows_the_ops_sees_the_modules():
     with torch.utils.flop_counter.FlopCounterMode(display=False):
         look(x)
     assert seen == [False, True, True, True, True]
+
+
+@pytest.mark.parametrize("change", ["bias type", "weight strides"])
+def test_norm_parameters_that_the_kernels_do_not_take(monkeypatch, change):
+    """Eager LayerNorm under autocast takes both."""
+    monkeypatch.setattr(torch, "is_autocast_enabled", lambda *a: True)
+    monkeypatch.setattr(torch, "get_autocast_dtype", lambda *a: torch.float16)
+
+    def spoil(norm):
+        if change == "bias type":
+            norm.bias = torch.nn.Parameter(norm.bias.float(), requires_grad=False)
+        else:
+            norm.weight = torch.nn.Parameter(norm.weight.repeat_interleave(2)[::2], requires_grad=False)
+
+    block = _block()
+    assert _fused(monkeypatch, block)
+    spoil(block.norm2)
+    assert not _fused(monkeypatch, block)
+
+    def called(self, x):
+        return "called"
+
+    merge = sw.PatchMerging(32).half().eval().requires_grad_(False)
+    monkeypatch.setattr(monai_patch, "patch_merge_3d", lambda *a: "fused")
+    x = torch.zeros((1, 4, 4, 4, 32), dtype=torch.float16)
+    assert monai_patch._downsample(merge, x, sw) == "fused"
+    spoil(merge.norm)
+    monkeypatch.setattr(sw.PatchMerging, "__call__", called)
+    assert monai_patch._downsample(merge, x, sw) == "called"
