@@ -297,6 +297,7 @@ def _patched_window_attention_forward(original):
 # ---- what the eager modules would do beyond the values ---------------------------
 
 _HALF = (torch.float16, torch.bfloat16)
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
 def _computes_half(x: torch.Tensor) -> bool:
@@ -353,10 +354,11 @@ def _values_only(x: torch.Tensor, params) -> bool:
 def _half_compute(x: torch.Tensor, params) -> torch.dtype | None:
     """The 16-bit type the Linears of ``params`` run in on ``x``, or None
     where they run in fp32, or where the eager ops mix types in another way
-    (without autocast everything must share x's type).  The kernels' 16-byte
-    accesses need what eager does not, aligned storage (parameters that are
-    views of one flat vector often are not)."""
-    if any(t.data_ptr() % 16 for t in (x, *params)):
+    (without autocast everything must share x's type).  Tensor subclasses
+    (quantised or distributed weights) bring ops of their own; the kernels'
+    16-byte accesses need what eager does not, aligned storage (parameters
+    that are views of one flat vector often are not)."""
+    if any(type(p) not in _PLAIN for p in params) or any(t.data_ptr() % 16 for t in (x, *params)):
         return None
     if torch.is_autocast_enabled("cuda"):
         dtype = torch.get_autocast_dtype("cuda")

@@ -225,3 +225,13 @@ def test_norm_parameters_that_the_kernels_do_not_take(monkeypatch, change):
     spoil(merge.norm)
     monkeypatch.setattr(sw.PatchMerging, "__call__", called)
     assert monai_patch._downsample(merge, x, sw) == "called"
+
+
+class _Weight(torch.Tensor):
+    pass
+
+
+def test_weights_of_a_tensor_subclass_keep_their_ops():
+    x = torch.zeros(8, dtype=torch.float16)
+    assert monai_patch._half_compute(x, [x.clone(), torch.nn.Parameter(x.clone())]) is torch.float16
+    assert monai_patch._half_compute(x, [torch.nn.Parameter(x.clone().as_subclass(_Weight))]) is None
