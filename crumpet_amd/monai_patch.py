@@ -461,7 +461,10 @@ def _patched_block_forward(original, swin):
         if dtype is None:
             return original(self, x, mask_matrix)
         half = self.forward_part1(x, mask_matrix)
-        if half.dtype != dtype:
+        # a gradient through the attention half (its parameters may train while
+        # the MLP's do not), or a half that a subclass gave another form
+        if (half.dtype != dtype or half.requires_grad or half.shape != x.shape or type(half) is not torch.Tensor
+                or half.data_ptr() % 16):
             x = x + half
             return x + self.forward_part2(x)
         return fused_swin_mlp(x, half, self.norm2, self.mlp.linear1, self.mlp.linear2, dtype)

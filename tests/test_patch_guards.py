@@ -235,3 +235,27 @@ def test_weights_of_a_tensor_subclass_keep_their_ops():
     x = torch.zeros(8, dtype=torch.float16)
     assert monai_patch._half_compute(x, [x.clone(), torch.nn.Parameter(x.clone())]) is torch.float16
     assert monai_patch._half_compute(x, [torch.nn.Parameter(x.clone().as_subclass(_Weight))]) is None
+
+
+@pytest.mark.parametrize("form", ["gradient", "broadcast", "unaligned"])
+def test_the_first_half_may_need_the_eager_second(monkeypatch, form):
+    """Parameters of the attention half that train in eval mode beside a
+    frozen MLP keep their gradients; other forms of its result are added as
+    eager adds them."""
+    def first_half(self, x, mask_matrix):
+        if form == "gradient":
+            return x * torch.ones(32, dtype=torch.float16, requires_grad=True)
+        if form == "broadcast":
+            return x[..., :1]
+        flat = torch.empty(x.numel() + 1, dtype=x.dtype)
+        return flat[1:].view(x.shape).copy_(x)
+
+    monkeypatch.setattr(monai_patch, "_tail_dtype", lambda *a: torch.float16)
+    monkeypatch.setattr(monai_patch, "fused_swin_mlp", lambda *a: pytest.fail("fused second half"))
+    crumpet_amd.patch_monai_swin_unetr()
+    try:
+        block = _block(type("Block", (sw.SwinTransformerBlock,), {"forward_part1": first_half}))
+        y = block(torch.randn((1, 2, 2, 2, 32)).half(), None)
+        assert y.shape == (1, 2, 2, 2, 32) and y.requires_grad == (form == "gradient")
+    finally:
+        crumpet_amd.unpatch_monai_swin_unetr()
