@@ -152,24 +152,54 @@ def _fused_block_supported(block, x: torch.Tensor) -> bool:
     return c % 16 == 0 and c <= 384 and _fits_staging_tile(c, _ESIZE[_compute_dtype(x)])
 
 
+class _Entry:
+    """A value that ``_cached`` keeps.  ``held`` are the source tensors'
+    storages: while they live no other tensor can be found at their
+    addresses.  Copies and pickles of a module start without the entry."""
+
+    __slots__ = ("stamp", "held", "value")
+
+    def __init__(self, stamp, sources, value):
+        self.stamp, self.value = stamp, value
+        self.held = tuple(t.detach() for t in sources)
+
+    def __deepcopy__(self, memo):
+        return None
+
+    def __reduce__(self):
+        return type(None), ()
+
+
 def _cached(module, key, sources, make):
     """``make()`` for ``key``, kept on ``module`` until a tensor in ``sources``
     changes: an in-place update bumps its version counter, reassigning it
-    changes its storage.  Under graph capture nothing is cached or reused:
-    the value is recomputed by kernels the graph records, so every replay
-    reads the parameters as they are then (the reference recomputes the bias
-    on every call for that reason, torch-ext/crumpet/monai_patch.py:157-162)."""
+    (also through ``.data``, or by a call that swaps parameters in) changes
+    its storage.  A write *into* ``.data`` does neither and is not seen;
+    ``forget_cached_params`` is for programs that write so.  Under graph
+    capture nothing is cached or reused: the value is recomputed by kernels
+    the graph records, so every replay reads the parameters as they are then
+    (the reference recomputes the bias on every call for that reason,
+    torch-ext/crumpet/monai_patch.py:157-162)."""
     if torch.cuda.is_available() and torch.cuda.is_current_stream_capturing():
         return make()
     stamp = tuple((t._version, t.data_ptr()) for t in sources)
     cache = module.__dict__.setdefault("_crumpet_cache", {})
     hit = cache.get(key)
-    if hit is not None and hit[0] == stamp:
-        return hit[1]
+    if hit is not None and hit.stamp == stamp:
+        return hit.value
     with torch.no_grad():
         value = make()
-    cache[key] = (stamp, value)
+    cache[key] = _Entry(stamp, sources, value)
     return value
+
+
+def forget_cached_params(model: torch.nn.Module) -> None:
+    """Drop what the patched attention half keeps of its parameters (the
+    gathered relative-position bias, the projections in the compute type), to
+    be made anew by the next pass: for programs that write into a
+    parameter's ``.data`` between passes, which nothing else shows."""
+    for module in model.modules():
+        module.__dict__.pop("_crumpet_cache", None)
 
 
 def _window_bias(attn, n):

@@ -3,6 +3,9 @@ channels-last chain for the eager modules (no GPU needed to decide that)."""
 
 from __future__ import annotations
 
+import copy
+import pickle
+
 import pytest
 import torch
 import torch.utils.flop_counter
@@ -259,3 +262,40 @@ def test_the_first_half_may_need_the_eager_second(monkeypatch, form):
         assert y.shape == (1, 2, 2, 2, 32) and y.requires_grad == (form == "gradient")
     finally:
         crumpet_amd.unpatch_monai_swin_unetr()
+
+
+def test_kept_parameters_are_not_known_by_a_reused_address():
+    """Parameters that every call swaps in start at version 0, and without
+    a hold on the last ones' storage land on the address that they left."""
+    attn = _Bias(sw.WindowAttention(48, 3, (4, 4, 4)))
+    shape = attn.attn.relative_position_bias_table.shape
+    for i in range(20):
+        table = torch.full(shape, float(i))
+        assert (torch.func.functional_call(attn, {"attn.relative_position_bias_table": table}, ()) == i).all()
+        del table
+
+
+class _Bias(torch.nn.Module):
+    def __init__(self, attn):
+        super().__init__()
+        self.attn = attn
+
+    def forward(self):
+        return monai_patch._window_bias(self.attn, 64)
+
+
+def test_writes_into_data_are_seen_after_forgetting():
+    block = _block(c=48)
+    first = monai_patch._window_bias(block.attn, 64).clone()
+    block.attn.relative_position_bias_table.data.add_(1)
+    monai_patch.forget_cached_params(block)
+    assert torch.equal(monai_patch._window_bias(block.attn, 64), first + 1)
+
+
+def test_copies_of_a_module_start_without_kept_parameters():
+    attn = sw.WindowAttention(48, 3, (4, 4, 4))
+    first = monai_patch._window_bias(attn, 64)
+    for other in (copy.deepcopy(attn), pickle.loads(pickle.dumps(attn))):
+        assert not any(other.__dict__["_crumpet_cache"].values())
+        other.relative_position_bias_table.data.add_(1)
+        assert torch.equal(monai_patch._window_bias(other, 64), first + 1)
