@@ -152,16 +152,37 @@ def _fused_block_supported(block, x: torch.Tensor) -> bool:
     return c % 16 == 0 and c <= 384 and _fits_staging_tile(c, _ESIZE[_compute_dtype(x)])
 
 
+def _tensors(value):
+    """The tensors of a value that ``_cached`` keeps."""
+    if isinstance(value, torch.Tensor):
+        return [value]
+    return [] if value is None else [t for v in value for t in _tensors(v)]
+
+
 class _Entry:
     """A value that ``_cached`` keeps.  ``held`` are the source tensors'
     storages: while they live no other tensor can be found at their
-    addresses.  Copies and pickles of a module start without the entry."""
+    addresses.  Another stream than the one that made the value waits for it,
+    and is noted with its memory.  Copies and pickles of a module start
+    without the entry."""
 
-    __slots__ = ("stamp", "held", "value")
+    __slots__ = ("stamp", "held", "value", "device", "stream", "made")
 
     def __init__(self, stamp, sources, value):
         self.stamp, self.value = stamp, value
         self.held = tuple(t.detach() for t in sources)
+        self.device, self.stream, self.made = sources[0].device, None, None
+        if self.device.type == "cuda":
+            current = torch.cuda.current_stream(self.device)
+            self.stream, self.made = current.cuda_stream, current.record_event()
+
+    def use(self):
+        if self.made is not None and torch._C._cuda_getCurrentRawStream(self.device.index) != self.stream:
+            current = torch.cuda.current_stream(self.device)
+            current.wait_event(self.made)
+            for t in _tensors(self.value):
+                t.record_stream(current)
+        return self.value
 
     def __deepcopy__(self, memo):
         return None
@@ -186,7 +207,7 @@ def _cached(module, key, sources, make):
     cache = module.__dict__.setdefault("_crumpet_cache", {})
     hit = cache.get(key)
     if hit is not None and hit.stamp == stamp:
-        return hit.value
+        return hit.use()
     with torch.no_grad():
         value = make()
     cache[key] = _Entry(stamp, sources, value)
