@@ -3,8 +3,8 @@
 // rows 16-byte aligned.  Contract, mask modes and numerics of
 // swin_attention_wide_kernel (attention_wide.hip): q scaled in fp32 and
 // rounded to the input type, scores and softmax in fp32, P rounded to the
-// input type for the P v product, one division at the end; the row sums run
-// over the rounded P, as in the bias-stationary kernel.
+// input type for the P v product, the row sums accumulated from the unrounded
+// fp32 P, one division at the end.
 //
 // Decomposition: a workgroup of 4 waves owns one (window, head) and 64 QT
 // queries, QT 16-query tiles per wave, and walks the keys in chunks of 64.
@@ -88,7 +88,11 @@ struct RowWords {
     }
 };
 
-// Max over the 4 lane groups (lanes l, l ^ 16, l ^ 32, l ^ 48).
+// Sum and max over the 4 lane groups (lanes l, l ^ 16, l ^ 32, l ^ 48).
+__device__ __forceinline__ float sum_groups(float x) {
+    x += __shfl_xor(x, 16);
+    return x + __shfl_xor(x, 32);
+}
 __device__ __forceinline__ float over_groups(float x) {
     uint32_t u = __float_as_uint(x);
     auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
@@ -244,20 +248,14 @@ swin_attention_chunk_kernel(const Params p, int32_t mask_dtype, uint32_t qblocks
     }
 
     f32x4 o[QT][kDT];  // o[i][dd][r] = O[query][16 dd + 4 g + r]
-    // every row of l[i]: the row sum of the query's rounded P (ones^T P^T), the
-    // values that the numerator uses, so that the rounding of a dominant P
-    // cancels
-    f32x4 l[QT];
+    float l[QT];       // this lane's share of the query's row sum (its keys), of the fp32 P
     float m_run[QT];
-    X8 ones;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) ones[e] = static_cast<T>(1.0f);
 #pragma unroll
     for (int i = 0; i < QT; ++i) {
 #pragma unroll
         for (int dd = 0; dd < kDT; ++dd) o[i][dd] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         m_run[i] = kLowestMax;
-        l[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        l[i] = 0.0f;
     }
     stash_kv(0);
     __syncthreads();  // chunk 0 and the class table are in LDS
@@ -373,10 +371,9 @@ swin_attention_chunk_kernel(const Params p, int32_t mask_dtype, uint32_t qblocks
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const float pv = __builtin_amdgcn_exp2f(__builtin_fmaf(S[i][2 * pr + u][r], kLog2e, -mb[i]));
+                        l[i] += pv;
                         pb[i][4 * u + r] = static_cast<T>(pv);
                     }
-#pragma unroll
-            for (int i = 0; i < QT; ++i) l[i] = F::mma32(ones, pb[i], l[i]);
             // O^T += V^T P^T: lane (col, g) holds V[keys 4 g .. of both tiles][16 dd + col]
             const int vrow = 32 * pr + 4 * g + (col >> 2);
 #pragma unroll
@@ -394,13 +391,14 @@ swin_attention_chunk_kernel(const Params p, int32_t mask_dtype, uint32_t qblocks
 
 #pragma unroll
     for (int i = 0; i < QT; ++i) {
+        const float sum = sum_groups(l[i]);
         if (qi[i] < N) {
             T* orow = static_cast<T*>(p.out) + int64_t(b) * p.os[0] + int64_t(h) * p.os[1] + int64_t(qi[i]) * p.os[2];
 #pragma unroll
             for (int dd = 0; dd < kDT; ++dd) {
                 X4 ov;
 #pragma unroll
-                for (int r = 0; r < 4; ++r) ov[r] = static_cast<T>(o[i][dd][r] / l[i][0]);
+                for (int r = 0; r < 4; ++r) ov[r] = static_cast<T>(o[i][dd][r] / sum);
                 *reinterpret_cast<X4*>(orow + 16 * dd + 4 * g) = ov;
             }
         }

@@ -9,6 +9,8 @@ of each other."""
 
 from __future__ import annotations
 
+import math
+
 import pytest
 import torch
 
@@ -81,3 +83,21 @@ def test_lowest_and_infinite_masks(dev, mask_dtype):
         mask[:, :, ~keep] = low
         got = fused_swin_attention(q, k, v, bias, mask)
         assert (got.double() - want).abs().max().item() <= TOL[torch.float16]
+
+
+@pytest.mark.parametrize("dtype,u", [(torch.float16, 2.0 ** -11), (torch.bfloat16, 2.0 ** -8)])
+@pytest.mark.parametrize("Dh,N", [(32, 400), (32, 512), (64, 343), (128, 343)])
+def test_row_sums_of_unrounded_probabilities(dev, dtype, u, Dh, N):
+    """One dominant key and equal small ones of a probability that 16 bits
+    round by almost u, with values of no weight: the row sum alone decides
+    the result, which is then off by its own rounding (u) and a few fp32
+    roundings.  A sum of the rounded probabilities would add almost another u."""
+    g = torch.Generator(device="cuda").manual_seed(Dh)
+    q = torch.zeros((2, 2, N, Dh), device="cuda", dtype=dtype)
+    v = torch.zeros_like(q)
+    v[:, :, 7] = (1 + torch.rand((2, 2, Dh), generator=g, device="cuda")).to(dtype)
+    bias = torch.full((2, N, N), math.log((1 + 0.98 * u) / 8), device="cuda")
+    bias[:, :, 7] = 0
+    got = fused_swin_attention(q, q, v, bias, None).double()
+    want = v[:, :, 7:8].double() / (1 + (N - 1) * bias[0, 0, 0].double().exp())
+    assert ((got - want).abs() / want).max().item() <= 1.05 * u
