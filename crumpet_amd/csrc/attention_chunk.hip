@@ -36,9 +36,12 @@ namespace {
 
 constexpr int kChunkKeys = 64;
 constexpr int kChunkThreads = 256;
-// The row max starts here: keys at -inf, or at the lowest value of fp32 or
-// bf16 (whose product with log2 e overflows), then have a P of 0.
-constexpr float kLowestMax = -1e38f;
+// The row max starts at the lowest float, so that keys at -inf have a P of 0.
+constexpr float kLowestMax = -3.402823466e38f;
+// Row maxima below this (rows masked wholly with the lowest value of fp32 or
+// bf16): the product with log2 e would overflow, and keys that differ at all
+// differ by more than 1e31, so that P is 1 at the max and 0 elsewhere.
+constexpr float kScaledMax = -1e38f;
 typedef uint32_t u32x3c __attribute__((ext_vector_type(3)));
 typedef uint32_t u32x4c __attribute__((ext_vector_type(4)));
 
@@ -359,7 +362,20 @@ swin_attention_chunk_kernel(const Params p, int32_t mask_dtype, uint32_t qblocks
             }
         }
 #pragma unroll
-        for (int i = 0; i < QT; ++i) mb[i] = m_run[i] * kLog2e;
+        for (int i = 0; i < QT; ++i) {
+            mb[i] = m_run[i] * kLog2e;
+            if (__any(m_run[i] < kScaledMax)) {
+                const bool low = m_run[i] < kScaledMax;
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        const float d = S[i][t][r] < m_run[i] ? -INFINITY : S[i][t][r] - m_run[i];
+                        S[i][t][r] = low ? d : S[i][t][r];
+                    }
+                mb[i] = low ? 0.0f : mb[i];
+            }
+        }
 
 #pragma unroll
         for (int pr = 0; pr < 2; ++pr) {

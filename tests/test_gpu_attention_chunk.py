@@ -101,3 +101,31 @@ def test_row_sums_of_unrounded_probabilities(dev, dtype, u, Dh, N):
     got = fused_swin_attention(q, q, v, bias, None).double()
     want = v[:, :, 7:8].double() / (1 + (N - 1) * bias[0, 0, 0].double().exp())
     assert ((got - want).abs() / want).max().item() <= 1.05 * u
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("Dh,N", [(32, 400), (32, 512), (64, 200), (128, 200)])
+@pytest.mark.parametrize("mask_dtype,low", [(torch.float32, torch.finfo(torch.float32).min),
+                                            (torch.bfloat16, torch.finfo(torch.bfloat16).min),
+                                            (torch.float32, -1.5e38)])
+def test_rows_masked_wholly_by_a_low_value(dev, dtype, Dh, N, mask_dtype, low):
+    """Every key of a row at the lowest value: the scores vanish in it (they do
+    not in fp16's, which leaves them 2^-8 steps of fp32) and the result is the mean of v, as of torch.softmax; with keys at -inf beside
+    them, the mean of the others; a row all at -inf is NaN."""
+    g = torch.Generator(device="cuda").manual_seed(2)
+    q, k, v = (torch.randn((1, 2, N, Dh), generator=g, device="cuda").to(dtype) for _ in range(3))
+    bias = torch.randn((2, N, N), generator=g, device="cuda")
+    mask = torch.zeros((1, N, N), dtype=mask_dtype, device="cuda")
+    mask[:, 3] = low
+    mask[:, 5] = low
+    mask[:, 5, ::3] = float("-inf")
+    mask[:, 6, :130] = low
+    mask[:, 7, 130:] = low
+    mask[:, 8] = float("-inf")
+    got = fused_swin_attention(q, k, v, bias, mask).double()
+    # the scores in fp32, where they vanish in the mask
+    s = ((q.double() * Dh ** -0.5) @ k.double().transpose(-2, -1).contiguous() + bias.double()).float()
+    want = torch.softmax((s + mask.float()[:, None]).double(), -1) @ v.double()
+    assert torch.isnan(got[:, :, 8]).all()
+    rows = torch.arange(N, device="cuda") != 8
+    assert (got - want)[:, :, rows].abs().max().item() <= TOL[dtype]
