@@ -218,8 +218,14 @@ int run_attention(const char* what, void* out, const int64_t out_strides[4], con
         if (((N - 1) * st[i][2] + 32) * esize >= (int64_t(1) << 31)) tuned32 = false;
     }
     // head dims 32, 64 and 128 of 16-bit types with 16-byte aligned q, k and
-    // v rows run the chunk kernel, the rest of `wide` the general one
-    if (wide && !tuned32 && vec && dtype != CRUMPET_DTYPE_F32 && (Dh == 32 || Dh == 64 || Dh == 128)) {
+    // v rows run the chunk kernel, the rest of `wide` the general one.  Head
+    // dim 32 with few keys stays with the latter, whose chunks are of 32 keys
+    // (64 there; fp16, 6 heads, chunk / general us: 1,616 windows of 27 29.8 /
+    // 25.9, 1,320 of 33 26.2 / 30.9; with a mask tensor 3,120 of 15 59.6 /
+    // 56.0, 2,728 of 16 55.7 / 58.7).
+    const int few_keys = Dh != 32 ? 0 : attn::mask_tensor(kmask) ? 15 : 32;
+    if (wide && !tuned32 && vec && dtype != CRUMPET_DTYPE_F32 && (Dh == 32 || Dh == 64 || Dh == 128) &&
+        N > few_keys) {
         bool rows16 = true;
         for (int i = 0; i < 3; ++i)
             if (st[i][0] % 8 || st[i][1] % 8 || st[i][2] % 8 || reinterpret_cast<uintptr_t>(ptr[i]) % 16)

@@ -129,3 +129,27 @@ def test_rows_masked_wholly_by_a_low_value(dev, dtype, Dh, N, mask_dtype, low):
     assert torch.isnan(got[:, :, 8]).all()
     rows = torch.arange(N, device="cuda") != 8
     assert (got - want)[:, :, rows].abs().max().item() <= TOL[dtype]
+
+
+def _formula(q, k, v, bias, mask):
+    s = (q.double() * q.shape[-1] ** -0.5) @ k.double().transpose(-2, -1).contiguous() + bias.double()
+    return torch.softmax(s if mask is None else s + mask.double()[:, None], -1) @ v.double()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("Dh,N", [(32, n) for n in (1, 15, 16, 31, 32, 33, 64, 65, 127, 128, 353, 385, 450, 512)]
+                         + [(d, n) for d in (64, 128) for n in (1, 16, 63, 64, 65, 129, 192, 353)])
+def test_few_and_many_keys_against_64_bits(dev, dtype, Dh, N):
+    """Both sides of the line below which head dim 32 stays with the general
+    kernel (16 keys with a mask tensor, 33 without), and of every chunk."""
+    g = torch.Generator(device="cuda").manual_seed(N)
+    q, k, v = (torch.randn((4, 2, N, Dh), generator=g, device="cuda").to(dtype) for _ in range(3))
+    bias = torch.randn((2, N, N), generator=g, device="cuda")
+    mask = torch.where(torch.rand((4, N, N), generator=g, device="cuda") < 0.3, -100.0, 0.0)
+    mask[:, :, N // 2] = 0
+    assert (fused_swin_attention(q, k, v, bias, None).double() - _formula(q, k, v, bias, None)).abs().max() <= TOL[dtype]
+    assert (fused_swin_attention(q, k, v, bias, mask).double() - _formula(q, k, v, bias, mask)).abs().max() <= TOL[dtype]
+    dims, ws, shift = (2, 2, N), (1, 1, N), (0, 0, N // 2)
+    region = crumpet_amd.compute_attn_mask_3d(*dims, ws, shift, torch.float32, "cuda")
+    got = fused_swin_attention_shifted(q, k, v, bias, dims, ws, shift)
+    assert (got.double() - _formula(q, k, v, bias, region)).abs().max() <= TOL[dtype]
