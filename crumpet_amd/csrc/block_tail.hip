@@ -248,7 +248,7 @@ __global__ void __launch_bounds__(256)
 rows_norm_kernel(To* __restrict__ out, Tx* __restrict__ sum_out, const Tx* __restrict__ x, const void* add,
                  int32_t add_dtype, const void* ln_w, const void* ln_b, int32_t ln_dtype, float eps, uint32_t T,
                  int32_t C, const MergeGeom m) {
-    const uint32_t t = blockIdx.x * (256 / LPR) + threadIdx.x / LPR;
+    const uint32_t t = (blockIdx.y * gridDim.x + blockIdx.x) * (256 / LPR) + threadIdx.x / LPR;
     const int part = threadIdx.x % LPR;
     const int nch = C >> 2;
     const uint32_t tr = t < T ? t : T - 1;
@@ -550,10 +550,13 @@ template <typename Tx, typename To, bool kMerge>
 void launch_norm(hipStream_t s, void* out, void* sum_out, const void* x, const void* add, int32_t add_dtype,
                  const void* ln_w, const void* ln_b, int32_t ln_dtype, float eps, uint32_t T, int32_t C,
                  const MergeGeom& m) {
-#define CRUMPET_NORM(L, V)                                                                                        \
-    hipLaunchKernelGGL((rows_norm_kernel<Tx, To, L, V, kMerge>), dim3((T + 256 / L - 1) / (256 / L)), dim3(256), 0, \
-                       s, static_cast<To*>(out), static_cast<Tx*>(sum_out), static_cast<const Tx*>(x), add,       \
-                       add_dtype, ln_w, ln_b, ln_dtype, eps, T, C, m)
+#define CRUMPET_NORM(L, V)                                                                                  \
+    do {                                                                                                    \
+        const GridXY g = grid_xy((T + 256 / L - 1) / (256 / L));                                            \
+        hipLaunchKernelGGL((rows_norm_kernel<Tx, To, L, V, kMerge>), dim3(g.x, g.y), dim3(256), 0, s,       \
+                           static_cast<To*>(out), static_cast<Tx*>(sum_out), static_cast<const Tx*>(x), add, \
+                           add_dtype, ln_w, ln_b, ln_dtype, eps, T, C, m);                                  \
+    } while (0)
     const int nch = C / 4;
     if (nch <= 4 * 3)
         CRUMPET_NORM(4, 3);

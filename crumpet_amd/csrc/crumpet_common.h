@@ -58,6 +58,22 @@ struct FastDiv {
 
 }  // namespace crumpet
 
+namespace crumpet {
+
+// HIP counts the threads of a launch along x in 32 bits.
+inline bool launch_takes(uint64_t workgroups, uint32_t threads) { return workgroups * threads < (uint64_t(1) << 32); }
+
+// A launch of `workgroups` over x and y; the last row of y may have idle ones.
+struct GridXY {
+    uint32_t x, y;
+};
+inline GridXY grid_xy(uint64_t workgroups) {
+    const uint64_t x = workgroups < (1u << 20) ? workgroups : (1u << 20);
+    return {static_cast<uint32_t>(x), static_cast<uint32_t>(x == 0 ? 0 : (workgroups + x - 1) / x)};
+}
+
+}  // namespace crumpet
+
 #if defined(__HIPCC__)
 
 namespace crumpet {

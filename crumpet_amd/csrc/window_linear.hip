@@ -1419,13 +1419,19 @@ bool rows_sizes(int32_t dtype, int64_t C) {
 // 17.9 against 18.1).
 constexpr int64_t kRowsMaxElements = int64_t(1) << 20;
 
+// Its workgroups: 64 features of 32 tokens each, all along x.  Past what a
+// launch takes (29.8 million tokens at 1,152 features) the other kernels run,
+// whose launches grow with the tokens alone.
+uint64_t rows_chunks(int64_t tokens, int64_t n_out) { return uint64_t((n_out + 63) / 64) * uint64_t((tokens + 31) / 32); }
+bool rows_launch(int64_t tokens, int64_t n_out) { return launch_takes(rows_chunks(tokens, n_out) + kNumXcd, kThreads); }
+
 template <typename Tx, typename Tc, bool kQkv>
 void launch_rows(hipStream_t s, void* out, const void* x, const void* ln_w, const void* ln_b, int32_t ln_dtype,
                  int32_t normalize, float eps, const void* w, const void* bias, int64_t C, int64_t n_out,
                  const WinGeom& g) {
     const uint32_t T = kQkv ? g.tokens : g.vtokens;
     const uint32_t ft = static_cast<uint32_t>((n_out + 63) / 64);
-    const uint32_t chunks = ft * ((T + 31) / 32);
+    const uint32_t chunks = static_cast<uint32_t>(rows_chunks(T, n_out));
 #define CRUMPET_ROWS(K)                                                                                      \
     hipLaunchKernelGGL((window_rows_kernel<Tx, Tc, K, kQkv>), dim3(xcd_launch_count(chunks)), dim3(kThreads), \
                        0, s, static_cast<Tc*>(out), static_cast<const Tx*>(x), ln_w, ln_b, ln_dtype,         \
@@ -1485,7 +1491,8 @@ extern "C" int crumpet_window_qkv_3d(void* out, int32_t dtype, const void* x, in
          reinterpret_cast<uintptr_t>(ln_weight) | reinterpret_cast<uintptr_t>(ln_bias)) % 16 != 0)
         return fail(CRUMPET_ERR_UNSUPPORTED, "%s: pointers must be 16-byte aligned", what);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (rows_sizes(dtype, C) && (!qkv_streams_lds(dtype, C, n_out) || g.tokens * C <= kRowsMaxElements)) {
+    if (rows_sizes(dtype, C) && rows_launch(g.tokens, n_out) &&
+        (!qkv_streams_lds(dtype, C, n_out) || g.tokens * C <= kRowsMaxElements)) {
         if (x_dtype == CRUMPET_DTYPE_F32)
             launch_rows_qkv<float>(dtype, s, out, x, ln_weight, ln_bias, ln_dtype, normalize, eps, weight, bias, C,
                                    n_out, g);
@@ -1555,7 +1562,7 @@ extern "C" int crumpet_window_proj_3d(void* y, const void* windows, int32_t dtyp
          reinterpret_cast<uintptr_t>(weight) | reinterpret_cast<uintptr_t>(bias)) % 16 != 0)
         return fail(CRUMPET_ERR_UNSUPPORTED, "%s: pointers must be 16-byte aligned", what);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (rows_sizes(dtype, C) && !proj_streams(dtype, C, n_out)) {
+    if (rows_sizes(dtype, C) && rows_launch(g.vtokens, n_out) && !proj_streams(dtype, C, n_out)) {
         if (dtype == CRUMPET_DTYPE_F16)
             launch_rows<_Float16, _Float16, false>(s, y, windows, nullptr, nullptr, CRUMPET_DTYPE_F32, 0, 0.0f,
                                                    weight, bias, C, n_out, g);

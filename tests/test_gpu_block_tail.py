@@ -258,3 +258,16 @@ def test_jit_trace_keeps_the_modules_parameters(dev):
         assert (got - want).abs().max().item() <= 6 * U[torch.float16] * want.abs().max().item()
 
     _patched(check)
+
+
+def test_channel_norm_over_more_rows_than_one_row_of_workgroups(dev):
+    """64 rows a workgroup and 2^20 workgroups along x: rows past 2^26."""
+    rows, c = (1 << 26) + 100, 8
+    x = torch.zeros((rows, c), device=dev, dtype=torch.float16)
+    parts = [slice(0, 1000), slice((1 << 26) - 1000, rows)]
+    for part in parts:
+        x[part] = torch.randn(x[part].shape, device=dev, dtype=torch.float16)
+    got = fused_block.channel_norm(x)
+    for part in parts:
+        want = F.layer_norm(x[part].double(), (c,))
+        assert (got[part].double() - want).abs().max().item() <= 2 * U[torch.float16] * want.abs().max().item()
