@@ -36,6 +36,7 @@ C_ABI_SYMBOLS = (
     "crumpet_window_proj_3d",
     "crumpet_swin_mlp",
     "crumpet_swin_mlp_fits",
+    "crumpet_cast_arrays",
     "crumpet_rows_norm",
     "crumpet_merge_norm_3d",
     "crumpet_rows_linear",

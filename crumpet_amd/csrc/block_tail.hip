@@ -229,6 +229,54 @@ swin_mlp_kernel(Tx* __restrict__ y, const Tx* __restrict__ x, const Tc* __restri
     }
 }
 
+// ---- fp32 parameters to the compute type ------------------------------------------
+
+// Up to four fp32 arrays into one buffer, each at the next multiple of 8
+// elements; a thread converts 8 (zeros past an array's end).  A launch and
+// the bytes bound it: 4.1 us for the MLP of 384 channels (1.2 million weights
+// and biases), where torch's foreach copy, in 20 workgroups of 64K elements,
+// takes 12.
+constexpr int kCastArrays = 4;
+struct CastArrays {
+    const float* src[kCastArrays];
+    uint32_t n[kCastArrays];      // elements
+    uint32_t first[kCastArrays];  // the array's first 8 elements in the buffer; unused ones past the end
+};
+
+template <typename Tc>
+__global__ void __launch_bounds__(256) cast_arrays_kernel(Tc* __restrict__ out, const CastArrays a, uint32_t total) {
+    typedef Tc T8 __attribute__((ext_vector_type(8)));
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= total) return;
+    int k = 0;
+#pragma unroll
+    for (int j = 1; j < kCastArrays; ++j) k = i >= a.first[j] ? j : k;
+    const float* src = a.src[0];
+    uint32_t n = a.n[0], first = a.first[0];
+#pragma unroll
+    for (int j = 1; j < kCastArrays; ++j)
+        if (k == j) {
+            src = a.src[j];
+            n = a.n[j];
+            first = a.first[j];
+        }
+    const uint32_t e0 = (i - first) * 8;
+    T8 v = {};
+    if (e0 + 8 <= n && reinterpret_cast<uintptr_t>(src) % 16 == 0) {
+        const f32x4 lo = *reinterpret_cast<const f32x4*>(src + e0), hi = *reinterpret_cast<const f32x4*>(src + e0 + 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            v[e] = static_cast<Tc>(lo[e]);
+            v[4 + e] = static_cast<Tc>(hi[e]);
+        }
+    } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            if (e0 + e < n) v[e] = static_cast<Tc>(src[e0 + e]);
+    }
+    *reinterpret_cast<T8*>(out + size_t(i) * 8) = v;
+}
+
 // ---- LayerNorm over rows or 2x2x2 neighbourhoods ---------------------------------
 
 // Neighbourhood rows: row (b, d, h, w) of the halved grid holds 8 parts of
@@ -664,6 +712,37 @@ extern "C" int crumpet_swin_mlp(void* y, const void* x, int32_t x_dtype, const v
 extern "C" int crumpet_swin_mlp_fits(int64_t C, int64_t hidden) {
     return C > 0 && C % 16 == 0 && C <= 16 * kMlpMaxKS && hidden > 0 && hidden % 32 == 0 && hidden <= (1 << 16) &&
            mlp_lds(static_cast<int>(C / 16), static_cast<int>(hidden / 16)) <= kMlpMaxLds;
+}
+
+extern "C" int crumpet_cast_arrays(void* out, int32_t dtype, const float* const* arrays, const int64_t* sizes,
+                                   int32_t count, void* stream) {
+    const char* what = "crumpet_cast_arrays";
+    if (esize_of(dtype) != 2) return fail(CRUMPET_ERR_UNSUPPORTED, "%s: dtype must be float16 or bfloat16", what);
+    if (count < 0 || count > kCastArrays || (count > 0 && (arrays == nullptr || sizes == nullptr)))
+        return fail(CRUMPET_ERR_INVALID_ARGUMENT, "%s: at most %d arrays", what, kCastArrays);
+    CastArrays a;
+    int64_t total = 0;
+    for (int i = 0; i < kCastArrays; ++i) {
+        a.src[i] = i < count ? arrays[i] : nullptr;
+        const int64_t n = i < count ? sizes[i] : 0;
+        if (n < 0 || (n > 0 && arrays[i] == nullptr))
+            return fail(CRUMPET_ERR_INVALID_ARGUMENT, "%s: negative size or null array", what);
+        if (n >= (int64_t(1) << 31)) return fail(CRUMPET_ERR_UNSUPPORTED, "%s: an array of 2^31 elements", what);
+        a.n[i] = static_cast<uint32_t>(n);
+        a.first[i] = i < count ? static_cast<uint32_t>(total) : 0xffffffffu;
+        total += (n + 7) / 8;
+    }
+    if (total == 0) return CRUMPET_OK;
+    if (out == nullptr) return fail(CRUMPET_ERR_INVALID_ARGUMENT, "%s: null output", what);
+    if (!aligned16({out})) return fail(CRUMPET_ERR_UNSUPPORTED, "%s: the output must be 16-byte aligned", what);
+    const uint32_t t = static_cast<uint32_t>(total);  // below 2^30
+    const dim3 grid((t + 255) / 256), block(256);
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (dtype == CRUMPET_DTYPE_F16)
+        hipLaunchKernelGGL((cast_arrays_kernel<_Float16>), grid, block, 0, s, static_cast<_Float16*>(out), a, t);
+    else
+        hipLaunchKernelGGL((cast_arrays_kernel<__bf16>), grid, block, 0, s, static_cast<__bf16*>(out), a, t);
+    return check_launch(what);
 }
 
 extern "C" int crumpet_rows_norm(void* out, int32_t out_dtype, void* sum_out, const void* x, int32_t x_dtype,

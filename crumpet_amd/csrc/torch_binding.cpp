@@ -17,7 +17,6 @@
 // C ABI of libcrumpet_hip.so (include/crumpet_hip.h).  A non-OK status
 // becomes a RuntimeError carrying crumpet_last_error().
 #include <ATen/core/Tensor.h>
-#include <ATen/ops/_foreach_copy.h>
 #include <ATen/ops/empty.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
@@ -26,7 +25,6 @@
 
 #include <array>
 #include <optional>
-#include <vector>
 
 #include "crumpet_hip.h"
 
@@ -524,36 +522,41 @@ int32_t norm_params(const std::optional<at::Tensor>& weight, const std::optional
 const void* ptr_or_null(const std::optional<at::Tensor>& t) { return t.has_value() ? t->data_ptr() : nullptr; }
 
 // Parameters of Linears in `dtype`: those that are in it already as they are,
-// the rest converted into one buffer (16-byte aligned pieces) by one launch.
-// On every call, so that a pass uses the parameters as they are then, however
-// they were written (a write through .data moves no version counter, and an
-// address is reused): about 9 us of host time for the four of an MLP, against
-// 20 for one conversion after the other.
+// fp32 ones converted into one buffer by one launch.  On every call, so that a
+// pass uses the parameters as they are then, however they were written (a
+// write through .data moves no version counter, and an address is reused).
 template <size_t N>
 std::array<std::optional<at::Tensor>, N> in_dtype(const std::array<const std::optional<at::Tensor>, N>& params,
-                                                  at::ScalarType dtype) {
+                                                  at::ScalarType dtype, const at::Device& dev) {
+    static_assert(N <= 4, "crumpet_cast_arrays takes four");
     at::AutoDispatchBelowADInplaceOrView below;
     std::array<std::optional<at::Tensor>, N> out;
-    std::vector<at::Tensor> from, to;
-    const int64_t align = 16 / static_cast<int64_t>(c10::elementSize(dtype));
-    int64_t size = 0;
+    std::array<at::Tensor, N> from;
+    const float* arrays[N];
+    int64_t sizes[N], total = 0;
+    int32_t count = 0;
     for (size_t i = 0; i < N; ++i) {
         if (!params[i].has_value()) continue;
-        out[i] = params[i]->scalar_type() == dtype ? params[i]->contiguous() : *params[i];
-        if (params[i]->scalar_type() != dtype) size += (params[i]->numel() + align - 1) / align * align;
+        const at::Tensor& p = *params[i];
+        if (p.scalar_type() == at::kFloat && dtype != at::kFloat && p.device() == dev) {
+            from[i] = p.contiguous();
+            arrays[count] = static_cast<const float*>(from[i].data_ptr());
+            sizes[count] = p.numel();
+            total += (sizes[count++] + 7) / 8 * 8;
+        } else {
+            out[i] = p.to(dtype).contiguous();
+        }
     }
-    if (size == 0) return out;
+    if (count == 0) return out;
     at::Tensor buffer;
     int64_t at = 0;
-    for (auto& t : out) {
-        if (!t.has_value() || t->scalar_type() == dtype) continue;
-        if (!buffer.defined()) buffer = at::empty({size}, t->options().dtype(dtype));
-        from.push_back(*t);
-        to.push_back(buffer.narrow(0, at, t->numel()).view(t->sizes()));
-        at += (t->numel() + align - 1) / align * align;
-        t = to.back();
+    for (size_t i = 0; i < N; ++i) {
+        if (!from[i].defined()) continue;
+        if (!buffer.defined()) buffer = at::empty({total}, from[i].options().dtype(dtype));
+        out[i] = buffer.as_strided(from[i].sizes(), from[i].strides(), at);
+        at += (from[i].numel() + 7) / 8 * 8;
     }
-    at::_foreach_copy_(to, from);
+    check_status(crumpet_cast_arrays(buffer.data_ptr(), dtype_code(dtype), arrays, sizes, count, stream_of(buffer)));
     return out;
 }
 
@@ -571,7 +574,7 @@ at::Tensor swin_mlp(const at::Tensor& x, const std::optional<at::Tensor>& add,
                 ": x must be a contiguous tensor on a HIP device");
     TORCH_CHECK(dtype_code(dtype) >= 0, what, ": dtype must be float32, float16 or bfloat16");
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
-    const auto params = in_dtype<4>({weight1, bias1, weight2, bias2}, dtype);
+    const auto params = in_dtype<4>({weight1, bias1, weight2, bias2}, dtype, x.device());
     const at::Tensor &w1 = *params[0], &w2 = *params[2];
     const std::optional<at::Tensor>&b1 = params[1], &b2 = params[3];
     const int64_t C = x.size(-1), rows = C > 0 ? x.numel() / C : 0;
@@ -619,7 +622,7 @@ at::Tensor patch_merge_3d(const at::Tensor& x, const std::optional<at::Tensor>& 
                 ": x must be a contiguous [B, D, H, W, C] tensor on a HIP device");
     TORCH_CHECK(dtype_code(dtype) >= 0, what, ": dtype must be float32, float16 or bfloat16");
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
-    const at::Tensor weight = *in_dtype<1>({reduction}, dtype)[0];
+    const at::Tensor weight = *in_dtype<1>({reduction}, dtype, x.device())[0];
     const int64_t B = x.size(0), D = x.size(1), H = x.size(2), W = x.size(3), C = x.size(4);
     const int32_t xdt = dtype_code(x.scalar_type()), dt = dtype_code(weight.scalar_type());
     TORCH_CHECK(xdt >= 0 && dt >= 0, what, ": dtypes must be float32, float16 or bfloat16");

@@ -360,6 +360,15 @@ CRUMPET_API int crumpet_swin_mlp(void* y, const void* x, int32_t x_dtype, const 
 CRUMPET_API int crumpet_swin_mlp_fits(int64_t C, int64_t hidden);
 
 /*
+ * Up to four fp32 arrays (any alignment) converted to `dtype` (float16 or
+ * bfloat16, round to nearest even) into out, each at the next multiple of 8
+ * elements, zeros between; out 16-byte aligned, of the sum of the sizes
+ * rounded up to 8.
+ */
+CRUMPET_API int crumpet_cast_arrays(void* out, int32_t dtype, const float* const* arrays, const int64_t* sizes,
+                                    int32_t count, void* stream);
+
+/*
  * out = LN(x) over rows of C channels, or with `add` x1 = x + add (written
  * to sum_out in x_dtype) and out = LN(x1).  out_dtype equals x_dtype or one
  * of the two is float32; LayerNorm in fp32, its parameters optional.  C a

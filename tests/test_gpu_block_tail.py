@@ -271,3 +271,28 @@ def test_channel_norm_over_more_rows_than_one_row_of_workgroups(dev):
     for part in parts:
         want = F.layer_norm(x[part].double(), (c,))
         assert (got[part].double() - want).abs().max().item() <= 2 * U[torch.float16] * want.abs().max().item()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("c,hidden", [(16, 32), (48, 192), (96, 384), (384, 1536)])
+@pytest.mark.parametrize("form", ["contiguous", "transposed", "4 bytes off", "one converted already"])
+def test_weights_converted_by_the_op(dev, dtype, c, hidden, form):
+    """The op's conversion of fp32 parameters against torch's, bit for bit,
+    through the results of the same kernels."""
+    g = torch.Generator().manual_seed(c)
+    x = _randn(g, 50, c)
+    norm = _norm(g, c, torch.float32)
+    w1, b1 = _randn(g, hidden, c, std=c ** -0.5), _randn(g, hidden, std=0.1)
+    w2, b2 = _randn(g, c, hidden, std=hidden ** -0.5), _randn(g, c, std=0.1)
+    u = U[dtype]
+    w1[0, :4] = torch.tensor([1 + u, 1 + 3 * u, -1e-7, 6.1e-5], device=dev)  # ties, fp16's smallest
+    if form == "transposed":
+        w1 = w1.t().contiguous().t()
+    elif form == "4 bytes off":
+        w2, b1 = (torch.empty(t.numel() + 1, device=dev)[1:].view(t.shape).copy_(t) for t in (w2, b1))
+    elif form == "one converted already":
+        w2 = w2.to(dtype)
+    got = fused_block.fused_swin_mlp(x, None, norm, (w1, b1), (w2, b2), dtype)
+    cast = [t.to(dtype).contiguous() for t in (w1, b1, w2, b2)]
+    want = fused_block.fused_swin_mlp(x, None, norm, cast[:2], cast[2:], dtype)
+    assert torch.isfinite(want).all() and torch.equal(got, want)
