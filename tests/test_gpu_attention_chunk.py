@@ -1,11 +1,14 @@
 """The chunk attention kernel (16-bit types, head dims 32, 64 and 128, rows
 16-byte aligned) against the general kernel, which the same values take when
 their rows lie 8 bytes off, at the edges of its chunks (64 keys, 64 or 128
-queries a workgroup) in every mask mode and bias type.
+queries a workgroup) in every mask mode and bias type, and against the formula
+in 64 bits.  At head dim 32, windows of 129 to 352 tokens run the tuned kernel
+and those of few keys the general one, whatever their alignment: there the
+first comparison is of that kernel with itself, and only the formula says more.
 
-Tolerance: the two differ in where P and the row sum are rounded; each is held
-to the type's bound against the fp32 formula (2e-3 / 1e-2), so to twice that
-of each other."""
+Tolerance: the two differ in the maxima that P is taken and rounded against;
+each is held to the type's bound against the formula (2e-3 / 1e-2), so to
+twice that of each other."""
 
 from __future__ import annotations
 
