@@ -1,6 +1,7 @@
 // Fused window attention in key chunks for 16-bit types at head dims 32, 64
-// and 128 (any N; head dim 32 where the bias-stationary kernel has no form),
-// rows 16-byte aligned.  Contract, mask modes and numerics of
+// and 128 (any N; at head dim 32 windows of more than 32 tokens, or 15 with a
+// mask tensor, where the bias-stationary kernel has no form), rows 16-byte
+// aligned.  Contract, mask modes and numerics of
 // swin_attention_wide_kernel (attention_wide.hip): q scaled in fp32 and
 // rounded to the input type, scores and softmax in fp32, P rounded to the
 // input type for the P v product, the row sums accumulated from the unrounded
@@ -19,7 +20,12 @@
 //   - One online-softmax update per chunk, the row max exact: the largest P
 //     is then 1 without rounding (a max that lags by up to 8 loses 20-30% of
 //     accuracy at sharp rows: 2.06e-3 against 1.7e-3 in fp16 at head dim 128).
-// The earlier form for these shapes (16 queries per wave, 16-deep products, a
+// VALU issue bounds it: 125 shifted windows of 343, 6 heads of 64, bf16 (84 us;
+// the general kernel 139) keep the VALU 69% busy, the matrix cores 14%, LDS
+// 22%, and the waves spend 29% of their cycles in waits; 128 windows of 512, 6
+// heads of 32, fp16 (109 us; 146) 50%, 9%, 7% and 29%, with 43% waiting to
+// issue.
+// The general kernel at these shapes (16 queries per wave, 16-deep products, a
 // transposing scalar store of V, one load per bias value) kept the matrix
 // cores at 6-7% of their rate, stalled on LDS stores and on 4-byte loads.
 #include <hip/hip_runtime.h>
@@ -437,16 +443,18 @@ void launch_q(const Params& p, int mode, int32_t mask_dtype, hipStream_t s) {
                            chunks);
 }
 
-// Two query tiles per wave at head dim 32 without a mask tensor, where
-// 128-query blocks pad N at most a fifth more than 64-query blocks: 112
-// against 123 us at N = 512 (128 windows x 6 heads).  Elsewhere the second
-// tile's registers cost a wave per SIMD and more than the shared fragments
-// give: 110 against 115 us there with a mask tensor, 82 against 85 us at head
-// dim 64, N = 343, 83 against 124 us at head dim 128.
+// Two query tiles per wave at head dim 32 without a mask tensor, for long
+// windows that 128-query blocks do not pad more than 64-query blocks, or that
+// are long enough for it not to matter.  fp16, 6 heads, us with one / two
+// tiles: 128 windows of 512 108 to 113 / 106, 40 of 1,000 121 / 112, 24 of
+// 1,536 199 / 177; but 336 of 128 26.6 / 29.2, 96 of 448 64 / 71, 72 of 576
+// 80 / 84.  Elsewhere the second tile's registers cost more than the shared
+// fragments give: 203 / 221 at 128 windows of 512 with a mask tensor, 129 /
+// 184 at head dim 128 (125 windows of 343); at head dim 64 they spill.
 template <typename T, int D>
 void launch_dim(const Params& p, int mode, int32_t mask_dtype, hipStream_t s) {
-    const int64_t n1 = (int64_t(p.N) + 63) / 64 * 64, n2 = (int64_t(p.N) + 127) / 128 * 128;
-    if (D == 32 && mode != 1 && 5 * n2 <= 6 * n1)
+    const bool even = (p.N + 63) / 64 % 2 == 0;
+    if (D == 32 && mode != 1 && p.N >= (even ? 512 : 700))
         launch_q<T, D, D == 32 ? 2 : 1>(p, mode, mask_dtype, s);
     else
         launch_q<T, D, 1>(p, mode, mask_dtype, s);

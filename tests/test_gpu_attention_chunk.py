@@ -140,7 +140,8 @@ def _formula(q, k, v, bias, mask):
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("Dh,N", [(32, n) for n in (1, 15, 16, 31, 32, 33, 64, 65, 127, 128, 353, 385, 450, 512)]
+@pytest.mark.parametrize("Dh,N", [(32, n) for n in (1, 15, 16, 31, 32, 33, 64, 65, 127, 128, 353, 385, 450, 511, 512,
+                                                    576, 640, 700, 729)]
                          + [(d, n) for d in (64, 128) for n in (1, 16, 63, 64, 65, 129, 192, 353)])
 def test_few_and_many_keys_against_64_bits(dev, dtype, Dh, N):
     """Both sides of the line below which head dim 32 stays with the general
