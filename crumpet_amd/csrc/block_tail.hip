@@ -120,10 +120,14 @@ __device__ __forceinline__ float gelu(float x) {
 //
 // Both weights live in LDS in fragment order (one conflict-free 8-byte read
 // per lane and product), filled once per workgroup; waves are independent
-// after that and take every waves-th tile.  The GELU (4 per lane and hidden
-// tile, about 60 issue cycles each wave) against 2 KS products of 8-16
-// cycles: the kernel is bound by VALU issue, not by the 6 bytes per channel
-// and token that it moves.
+// after that and take every waves-th tile.  What bounds it (fp16, counters of
+// one encoder pass): at 48 channels and 110,592 tokens (33 us, 1.0 TB/s) the
+// VALU is 43% busy, mostly with the GELU (4 per lane and hidden tile, about 60
+// issue cycles each wave, against 2 KS products of 8 to 16), and the waves
+// wait half of their cycles on the fill and the rows, for two tiles each.  At
+// 96 channels and 13,824 tokens (24 us) the 146 KB of weights leave one
+// workgroup a CU: one tile a wave behind the fill, one wave a SIMD, the VALU
+// 18% busy and 60% of the cycles waits.
 template <typename Tx, typename Tc, int KS>
 __global__ void __launch_bounds__(256)
 swin_mlp_kernel(Tx* __restrict__ y, const Tx* __restrict__ x, const Tc* __restrict__ add, const void* ln_w,
@@ -660,7 +664,14 @@ void launch_linear(hipStream_t s, void* out, const void* x, const void* w, const
                    int32_t act, uint32_t T, int32_t K, int32_t n_out) {
     const auto up = [](uint32_t a, uint32_t b) { return (a + b - 1) / b; };
     const uint32_t ft = up(static_cast<uint32_t>(n_out), 64);
-#define CRUMPET_LINEAR(BT, S)                                                                                 do {                                                                                                          const uint32_t chunks = ft * up(T, BT);                                                                   hipLaunchKernelGGL((rows_linear_kernel<Tc, To, BT, S>), dim3(xcd_launch_count(chunks)), dim3(256),                            0, s, static_cast<To*>(out), static_cast<const Tc*>(x),                                                   static_cast<const Tc*>(w), static_cast<const Tc*>(bias),                                                  static_cast<const To*>(res), act, T, K, n_out, ft, chunks);                        } while (0)
+#define CRUMPET_LINEAR(BT, S)                                                                              \
+    do {                                                                                                   \
+        const uint32_t chunks = ft * up(T, BT);                                                            \
+        hipLaunchKernelGGL((rows_linear_kernel<Tc, To, BT, S>), dim3(xcd_launch_count(chunks)), dim3(256), \
+                           0, s, static_cast<To*>(out), static_cast<const Tc*>(x),                         \
+                           static_cast<const Tc*>(w), static_cast<const Tc*>(bias),                        \
+                           static_cast<const To*>(res), act, T, K, n_out, ft, chunks);                     \
+    } while (0)
     // 64-token tiles once there are about three for every four CUs (216 x 768
     // -> 3072, 192 tiles: 8.5 us against 9.5 with 16-token tiles; 1,728 x
     // 1536 -> 384, 162 tiles: 13.0 against 12.0)

@@ -583,9 +583,9 @@ def _channels_last_chain(model, x, normalize, swin) -> bool:
     """Whether the encoder's stages may hand each other channels-last
     volumes: inference on plain tensors, the module's own ``proj_out``, every
     stage the patched ``BasicLayer`` without hooks, normalised features."""
-    if (torch.compiler.is_compiling() or model.training or not normalize or x.dim() != 5 or type(model) is not swin.SwinTransformer
-            or getattr(model, "use_v2", False) or not _stock(model, swin.SwinTransformer, "proj_out")
-            or not _fused_block_enabled()):
+    if (torch.compiler.is_compiling() or model.training or not normalize or x.dim() != 5
+            or type(model) is not swin.SwinTransformer or getattr(model, "use_v2", False)
+            or not _stock(model, swin.SwinTransformer, "proj_out") or not _fused_block_enabled()):
         return False
     layers = [getattr(model, f"layers{i + 1}", ()) for i in range(model.num_layers)]
     if swin.BasicLayer.forward is not _STATE.get("basic_layer", {}).get(swin.BasicLayer):
