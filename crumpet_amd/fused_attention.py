@@ -14,7 +14,7 @@ copies are needed) and writes ``out`` through its strides.  ``block_m`` and
 fixed by the MFMA shape (16-query strips, 16-key tiles).  Head dim 16 with
 up to 512 tokens per window (every Swin UNETR stage) runs the tuned kernel;
 16-bit inputs at head dims 32, 64 and 128 with 16-byte aligned rows run the
-chunk kernel, and the rest the general kernel (the head dims the reference's
+chunk kernel (at head dim 32 where the windows are not small), and the rest the general kernel (the head dims the reference's
 Triton kernel takes: powers of two from 16).
 """
 
