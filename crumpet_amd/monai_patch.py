@@ -453,10 +453,15 @@ def _norm_params(norm):
     return [p for p in (norm.weight, norm.bias) if p is not None]
 
 
-def _fusable_heads(attn) -> bool:
-    """Whether the attention runs fused.  Models whose head dimension is not
-    covered keep every other eager op too, and with them eager's exact bits."""
-    return _fused_attn_enabled() and attn.dim // attn.num_heads in _HEAD_DIMS and attn.attn_drop.p == 0.0
+def _fusable_heads(block) -> bool:
+    """Whether the block's attention runs fused.  Models whose head dimension
+    is not covered keep every other eager op too, and with them eager's exact
+    bits, and so do those whose blocks are something else."""
+    attn = getattr(block, "attn", None)
+    dim, heads, drop = (getattr(attn, name, None) for name in ("dim", "num_heads", "attn_drop"))
+    if dim is None or heads is None or drop is None:
+        return False
+    return _fused_attn_enabled() and dim // heads in _HEAD_DIMS and getattr(drop, "p", None) == 0.0
 
 
 @functools.lru_cache(maxsize=64)
@@ -480,7 +485,7 @@ def _tail_dtype(block, x, swin=None) -> torch.dtype | None:
         from . import swin_unetr_compat as swin
     if not _stock(block, swin.SwinTransformerBlock, "forward_part2"):
         return None
-    if getattr(block, "use_checkpoint", False) or not _fusable_heads(block.attn):
+    if getattr(block, "use_checkpoint", False) or not _fusable_heads(block):
         return None
     norm, mlp, c = block.norm2, block.mlp, x.shape[-1]
     # MONAI's swin_unetr imports its MLPBlock as Mlp
@@ -563,7 +568,7 @@ def _layer_channels_last(layer, x, swin):
         x = blk(x, attn_mask)
     x = x.view(b, d, h, w, -1)
     if layer.downsample is not None:
-        fused = len(layer.blocks) > 0 and _fusable_heads(layer.blocks[-1].attn)
+        fused = len(layer.blocks) > 0 and _fusable_heads(layer.blocks[-1])
         x = _downsample(layer.downsample, x, swin) if fused else layer.downsample(x)
     return x
 
@@ -591,7 +596,7 @@ def _channels_last_chain(model, x, normalize, swin) -> bool:
     if swin.BasicLayer.forward is not _STATE.get("basic_layer", {}).get(swin.BasicLayer):
         return False
     if not all(len(m) >= 1 and type(m[0]) is swin.BasicLayer and _unhooked(m[0]) and len(m[0].blocks)
-               and _fusable_heads(m[0].blocks[0].attn) for m in layers):
+               and _fusable_heads(m[0].blocks[0]) for m in layers):
         return False
     return _values_only(x, model.parameters())
 

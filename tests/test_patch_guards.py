@@ -299,3 +299,23 @@ def test_copies_of_a_module_start_without_kept_parameters():
         assert not any(other.__dict__["_crumpet_cache"].values())
         other.relative_position_bias_table.data.add_(1)
         assert torch.equal(monai_patch._window_bias(other, 64), first + 1)
+
+
+class _Plain(torch.nn.Module):
+    """A block of a program's own, without attention."""
+
+    def forward(self, x, mask_matrix):
+        return x + 1
+
+
+def test_stages_of_other_blocks_run(monkeypatch):
+    monkeypatch.setattr(monai_patch, "compute_attn_mask_3d", lambda **k: torch.zeros(1))
+    crumpet_amd.patch_monai_swin_unetr()
+    try:
+        model = _encoder()
+        assert _chained(monkeypatch, model)
+        model.layers1[0].blocks[0] = _Plain()
+        assert not _chained(monkeypatch, model)
+        assert model.layers1[0](torch.zeros((1, 32, 8, 8, 8))).shape == (1, 64, 4, 4, 4)
+    finally:
+        crumpet_amd.unpatch_monai_swin_unetr()
