@@ -457,11 +457,11 @@ def _fusable_heads(block) -> bool:
     """Whether the block's attention runs fused.  Models whose head dimension
     is not covered keep every other eager op too, and with them eager's exact
     bits, and so do those whose blocks are something else."""
-    attn = getattr(block, "attn", None)
-    dim, heads, drop = (getattr(attn, name, None) for name in ("dim", "num_heads", "attn_drop"))
-    if dim is None or heads is None or drop is None:
+    try:
+        attn = block.attn
+        return _fused_attn_enabled() and attn.dim // attn.num_heads in _HEAD_DIMS and attn.attn_drop.p == 0.0
+    except AttributeError:
         return False
-    return _fused_attn_enabled() and dim // heads in _HEAD_DIMS and getattr(drop, "p", None) == 0.0
 
 
 @functools.lru_cache(maxsize=64)
@@ -568,7 +568,7 @@ def _layer_channels_last(layer, x, swin):
         x = blk(x, attn_mask)
     x = x.view(b, d, h, w, -1)
     if layer.downsample is not None:
-        fused = len(layer.blocks) > 0 and _fusable_heads(layer.blocks[-1])
+        fused = _computes_half(x) and len(layer.blocks) > 0 and _fusable_heads(layer.blocks[-1])
         x = _downsample(layer.downsample, x, swin) if fused else layer.downsample(x)
     return x
 
