@@ -219,10 +219,11 @@ def test_second_half_and_merging_follow_their_weights(dev):
         agree(*both(lambda: {n: p * (1 + 0.2 * i) for n, p in start.items()}))
 
 
-def test_captured_second_half_reads_the_weights_at_replay(dev):
+@pytest.mark.parametrize("c", [48, 96, 192])  # one kernel, one with more than 64 KB of LDS, three kernels
+def test_captured_second_half_reads_the_weights_at_replay(dev, c):
     torch.manual_seed(0)
-    block = sw.SwinTransformerBlock(48, 3, (4, 4, 4), (0, 0, 0)).to(dev).eval().requires_grad_(False)
-    x = torch.randn((1, 8, 8, 8, 48), device=dev)
+    block = sw.SwinTransformerBlock(c, c // 16, (4, 4, 4), (0, 0, 0)).to(dev).eval().requires_grad_(False)
+    x = torch.randn((1, 8, 8, 8, c), device=dev)
 
     def run():
         with torch.no_grad(), torch.autocast("cuda", dtype=torch.float16, cache_enabled=False):
